@@ -335,7 +335,7 @@ const char* fa_strerror(int32_t code) {
         case FA_ERR_STRIDE: return "the d stride must be 1 and the b/s/h strides multiples of 16 bytes";
         case FA_ERR_HEADS: return "num_heads must be a positive multiple of num_heads_kv";
         case FA_ERR_DROPOUT: return "dropout_p must be in [0, 1)";
-        case FA_ERR_WORKSPACE: return "workspace is NULL or smaller than fa_bwd_workspace_size";
+        case FA_ERR_WORKSPACE: return "workspace is NULL or smaller than fa_fwd_workspace_size / fa_bwd_workspace_size";
         case FA_ERR_ALIGN: return "tensor base pointers must be 16-byte aligned";
         case FA_ERR_SCALE: return "scale must be finite and > 0";
         case FA_ERR_LAUNCH: return "the HIP runtime rejected a kernel launch";
@@ -376,11 +376,94 @@ int32_t fa_fwd_check(const fa_fwd_args* a) {
     return check_bias(a->bias, a->bias_stride, a->bias_dtype, a->dtype, a->seqlen_q, a->seqlen_k);
 }
 
-int32_t fa_fwd(const fa_fwd_args* a, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// Whether the few-row forward (csrc/fa_fwd_decode.hpp) runs, and into how many
+// key splits: 16-bit inputs, no bias or dropout.  Its units are 32-row tiles of
+// one (batch, KV head), each of which reads the keys for itself, so it wins
+// where the units (times the splits) fit the chip at once, and for a single
+// row tile (all rows of a KV head) at any count.  Measured against fwd_kernel /
+// fwd_pp_kernel (time ratio, bf16, (units; keys)):
+//   one generation: D = 128 causal (32; 1000) 0.64, (256; 1000) 0.61, (256;
+//   512) 0.67, (256; 256) 0.77, (192; 128) 0.93, (128; 8192 not causal) 0.34;
+//   D = 64 (64; 512) 0.67, (512; 2048) 0.66-0.83, (256; 256) 0.77, (512; 512)
+//   0.88-0.94, but (512; 128) 1.08 and (384; 192) 1.01: two workgroups on a CU
+//   need some keys to pay; D = 32 (512; 128) 0.86
+//   past one generation: D = 128 (384; 512) 1.13, (512; 1000) 1.07, but causal
+//   (512; 2048) 0.82 and (512; 4096) 0.79; D = 64 (768; 1024) 1.18, causal
+//   (1024; 4096) 0.75
+//   one row tile: D = 128 (384; 2000 keys, 4 heads a group) 0.44, D = 64 (800;
+//   6000, 1 head) 0.88-0.94, but (2048; 512, 32 queries of 1 head) 1.04
+bool decode_plan(const fa_fwd_args* a, fa::FwdParams& p) {
+    if (a->dtype == FA_DTYPE_F32 || a->head_dim > 128 || a->bias || a->dropout_p > 0.f) return false;
+    const bool causal = a->causal != 0;
+    const int D = a->head_dim;
+    const int64_t rows = (int64_t)(a->num_heads / a->num_heads_kv) * a->seqlen_q;
+    const int64_t keys = causal ? std::min(a->seqlen_q, a->seqlen_k) : a->seqlen_k;  // that the last query sees
+    const int64_t n_rt = (rows + 31) / 32;
+    // (rows x batch x KV heads below 2^30 here: no product of this plan overflows)
+    if (rows > (1 << 14) || (int64_t)a->batch * a->num_heads_kv > (1 << 16)) return false;
+    const int64_t units = n_rt * a->num_heads_kv * a->batch;
+    // workgroups that the LDS of 256 CUs holds at once (D = 32: as D = 64)
+    const int64_t slots = D == 128 ? 256 : 512;
+    const int64_t long_keys = D == 128 ? 2048 : 4096;
+    bool run = false;
+    if (units <= slots)
+        run = keys >= (D == 128 ? 192 : 65) && (D != 64 || units <= slots / 2 || keys >= 384);
+    else if (causal)
+        run = units <= 2 * slots && keys >= long_keys;
+    else
+        run = n_rt == 1 && keys >= (a->num_heads > a->num_heads_kv ? 256 : 1024);
+    if (!run) return false;
+    // the split count with the shortest run, estimated (in us) as the longer of
+    // the fullest CU's K / V bytes at its share of the memory bandwidth (0.8 us
+    // per 64 keys at D = 64; row tiles of one KV head share them through L2)
+    // and the chain of tiles per wave (about 1 us each, 3 us around them) over
+    // the generations of workgroups, plus the combining kernel.  Measured
+    // (one query, D = 64, 41 sequences of 1705 keys, 8 heads: 328 units, whose
+    // workgroups leave 72 CUs with two and the others with one): 1 split 41.6
+    // us, 3 splits 38.1 (fwd_kernel 41.0)
+    const int64_t nt = (keys + 63) / 64;
+    const double tb = 0.8 * D / 64 / (double)std::min<int64_t>(n_rt, 4);
+    int best = 1;
+    double best_cost = 1e30;
+    for (int ns = 1; ns <= 64 && (ns == 1 || ns * 8 <= nt); ++ns) {
+        const int64_t wgs = units * ns;
+        const int64_t per_wave = ((nt + ns - 1) / ns + 3) / 4;
+        const double bytes = (double)((wgs + 255) / 256) * (double)nt / ns * tb;
+        const double chain = (double)((wgs + slots - 1) / slots) * (double)(per_wave + 3);
+        const double cost = std::max(bytes, chain) + (ns > 1 ? 4.0 : 0.0);
+        if (cost < best_cost * 0.98) {
+            best_cost = cost;
+            best = ns;
+        }
+    }
+    p.dec_rt = (int)n_rt;
+    p.dec_splits = best;
+    return true;
+}
+// rows of the splits' parts (0 without a split) and their bytes
+size_t decode_part_rows(const fa_fwd_args* a, const fa::FwdParams& p) {
+    return p.dec_splits > 1 ? (size_t)a->batch * a->num_heads_kv * p.dec_rt * p.dec_splits * 32 : 0;
+}
+size_t decode_ws_bytes(const fa_fwd_args* a, const fa::FwdParams& p) {
+    return decode_part_rows(a, p) * (4 + (size_t)a->head_dim) * sizeof(float);
+}
+
+// fa_fwd; with a workspace of fa_fwd_workspace_size bytes, the few-row path
+// where decode_plan takes it
+int32_t fwd_run(const fa_fwd_args* a, void* ws, size_t ws_bytes, bool allow_split, void* stream) {
     int32_t st = fa_fwd_check(a);
     if (st) return st;
     if ((int64_t)a->batch * a->num_heads * a->seqlen_q == 0) return FA_OK;
     fa::FwdParams p{};
+    if (allow_split && decode_plan(a, p) && p.dec_splits > 1) {
+        if (!ws || !aligned16(ws) || ws_bytes < decode_ws_bytes(a, p)) return FA_ERR_WORKSPACE;
+        p.dec_stat = (float*)ws;
+        p.dec_part = p.dec_stat + decode_part_rows(a, p) * 4;
+    }
     p.q = a->q;
     p.k = a->k;
     p.v = a->v;
@@ -441,6 +524,26 @@ int32_t fa_fwd(const fa_fwd_args* a, void* stream) {
                                   : fa::launch_fwd_f16(p, a->head_dim, causal, dropout, s));
         default: return status_of(fa::launch_fwd_f32(p, a->head_dim, causal, dropout, s));
     }
+}
+
+}  // namespace
+
+extern "C" {
+
+int32_t fa_fwd(const fa_fwd_args* a, void* stream) { return fwd_run(a, nullptr, 0, false, stream); }
+
+size_t fa_fwd_workspace_size(const fa_fwd_args* a) {
+    if (!a) return 0;
+    if (check_common(a->batch, a->seqlen_q, a->seqlen_k, a->num_heads, a->num_heads_kv, a->head_dim, a->dtype,
+                     a->scale, a->dropout_p))
+        return 0;
+    fa::FwdParams p{};
+    if ((int64_t)a->batch * a->num_heads * a->seqlen_q == 0 || !decode_plan(a, p)) return 0;
+    return decode_ws_bytes(a, p);
+}
+
+int32_t fa_fwd_ws(const fa_fwd_args* a, void* workspace, size_t ws_bytes, void* stream) {
+    return fwd_run(a, workspace, ws_bytes, true, stream);
 }
 
 size_t fa_bwd_workspace_size(const fa_bwd_args* a) {

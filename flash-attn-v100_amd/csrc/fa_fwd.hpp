@@ -954,8 +954,15 @@ hipError_t launch_fwd_t(const FwdParams& p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The few-row forward (fa_fwd_decode.hpp, instantiated in fa_fwd_decode.hip)
+template <typename T>
+hipError_t launch_fwd_decode(const FwdParams& p, int D, bool causal, hipStream_t s);
+
 template <typename T, typename TB>
 hipError_t launch_fwd_dispatch(const FwdParams& p, int D, bool causal, bool dropout, hipStream_t s) {
+    if constexpr (!Elem<T>::kF32 && std::is_void<TB>::value) {
+        if (p.dec_splits > 0) return launch_fwd_decode<T>(p, D, causal, s);
+    }
     // dropout mode: 0 none, 1 Philox mask, 2 Philox mask also written as keep bits
     const int mode = !dropout ? 0 : (p.kb != nullptr ? 2 : 1);
 #define FA_FWD_MODES(DD, CC)                                                \

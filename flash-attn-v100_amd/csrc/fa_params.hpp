@@ -36,6 +36,14 @@ struct FwdParams {
     const void* bias;
     int64_t bias_sb, bias_sh, bias_ss;
     int bias_span;  // bytes of one (batch, head) slice: ((Sq - 1) * ss + Sk) * elem
+    // few-row forward (fa_fwd_decode.hpp), taken when dec_splits > 0: its units
+    // are the 32-row tiles of the (query head of the group, query) rows of each
+    // (batch, KV head), dec_rt per (batch, KV head); with dec_splits > 1 the
+    // parts of a unit's key splits go to the caller's workspace (per row 4
+    // floats of statistics, and D floats of O)
+    int dec_splits, dec_rt;
+    float* dec_stat;
+    float* dec_part;
 };
 
 struct BwdParams {

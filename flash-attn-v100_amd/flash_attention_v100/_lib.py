@@ -74,7 +74,8 @@ class BwdArgs(ctypes.Structure):
 
 
 EXPORTS = (
-    "fa_abi_version", "fa_strerror", "fa_fwd_check", "fa_fwd", "fa_bwd_workspace_size",
+    "fa_abi_version", "fa_strerror", "fa_fwd_check", "fa_fwd", "fa_fwd_workspace_size", "fa_fwd_ws",
+    "fa_bwd_workspace_size",
     "fa_bwd_check", "fa_bwd", "fa_bwd_stage", "fa_bwd_static", "fa_dropout_mask", "fa_rand",
 )
 
@@ -107,6 +108,10 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fa_fwd_check.argtypes = [P(FwdArgs)]
     lib.fa_fwd.restype = ctypes.c_int32
     lib.fa_fwd.argtypes = [P(FwdArgs), ctypes.c_void_p]
+    lib.fa_fwd_workspace_size.restype = ctypes.c_size_t
+    lib.fa_fwd_workspace_size.argtypes = [P(FwdArgs)]
+    lib.fa_fwd_ws.restype = ctypes.c_int32
+    lib.fa_fwd_ws.argtypes = [P(FwdArgs), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
     lib.fa_bwd_workspace_size.restype = ctypes.c_size_t
     lib.fa_bwd_workspace_size.argtypes = [P(BwdArgs)]
     lib.fa_bwd_check.restype = ctypes.c_int32
@@ -335,7 +340,9 @@ def fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: 
     if keep_bits is not None:
         _check_keep_bits(keep_bits, B, H, Sq, k.shape[1], q.device)
     a = fwd_args(q, k, v, o, lse, mx, causal, scale, dropout_p, seed, offset, pb, keep_bits)
-    _check("fa_fwd", lib.fa_fwd(ctypes.byref(a), _stream(q)))
+    ws_bytes = lib.fa_fwd_workspace_size(ctypes.byref(a))
+    ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
+    _check("fa_fwd_ws", lib.fa_fwd_ws(ctypes.byref(a), ws.data_ptr() if ws_bytes else None, ws_bytes, _stream(q)))
     return _unpad_d(o, D), lse, mx
 
 

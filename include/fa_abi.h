@@ -64,7 +64,7 @@ extern "C" {
 #define FA_ERR_STRIDE -5      /* d stride != 1, or b/s/h stride not a multiple of 16 bytes */
 #define FA_ERR_HEADS -6       /* num_heads not a positive multiple of num_heads_kv */
 #define FA_ERR_DROPOUT -7     /* dropout_p not in [0, 1) */
-#define FA_ERR_WORKSPACE -8   /* workspace NULL or smaller than fa_bwd_workspace_size */
+#define FA_ERR_WORKSPACE -8   /* workspace NULL or smaller than fa_{fwd,bwd}_workspace_size */
 #define FA_ERR_ALIGN -9       /* a tensor base pointer is not 16-byte aligned */
 #define FA_ERR_SCALE -10      /* scale not finite and > 0 */
 #define FA_ERR_LAUNCH -11     /* the HIP runtime rejected a kernel launch */
@@ -188,6 +188,19 @@ int32_t fa_fwd_check(const fa_fwd_args* args);
 /* Forward: o, lse (and max_vals if non-NULL).  Replaces
  * kernels/forward_kernel.py:246-387 (launch at :349-385). */
 int32_t fa_fwd(const fa_fwd_args* args, void* hip_stream);
+
+/* Bytes of device workspace fa_fwd_ws needs: for few query rows over many
+ * keys (16-bit inputs, no causal mask, bias or dropout) the keys may be split
+ * over several workgroups, whose float32 parts of every row go there; 0 where
+ * none is needed and on invalid arguments.  Host-only.  No reference
+ * counterpart. */
+size_t fa_fwd_workspace_size(const fa_fwd_args* args);
+
+/* fa_fwd with a workspace of at least fa_fwd_workspace_size bytes (NULL where
+ * that is 0; 16-byte aligned device memory, free again when the call's work on
+ * hip_stream has run): the same results, up to the order of the float32 sums
+ * where the keys are split.  FA_ERR_WORKSPACE if it is missing or too small. */
+int32_t fa_fwd_ws(const fa_fwd_args* args, void* workspace, size_t workspace_bytes, void* hip_stream);
 
 /* Bytes of device workspace fa_bwd needs: B * H rows of 2 * sq_pad float32
  * (sq_pad = Sq rounded up to 128; LSE * log2 e then delta = rowsum(dO * O),
