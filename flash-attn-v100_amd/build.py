@@ -23,18 +23,21 @@ OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "flash_attention_v100", "libfa_gfx950.so")
 ARCH = "gfx950"
 
+_H, _A = ("bf16", "f16"), ("bf16", "f16", "f32")
+_MODES = (("d256_", _H), ("cols_", _H), ("", _A), ("bias_", _A), ("bias32_", _H))
 SOURCES = ["fa_abi.cpp", "fa_misc.hip", "fa_fwd_fit.hip", "fa_fwd_decode.hip"] + [
     f"fa_{pas}_{mode}{dt}.hip"
-    for pas in ("bwd", "fwd")  # the backward units take longest: start them first
-    for mode, dts in (("d256_", ("bf16", "f16")), ("", ("bf16", "f16", "f32")), ("bias_", ("bf16", "f16", "f32")),
-                      ("bias32_", ("bf16", "f16")))
+    # the backward units take longest: start them first
+    for pas, modes in (("bwd", _MODES + (("cols256_", _H),)), ("fwd", _MODES))
+    for mode, dts in modes
     for dt in dts
 ]
 
 # units whose MFMA accumulators may live in AGPRs (the head-dim-256 backward:
 # its dK / dV and dQ kernels need more than 256 registers a lane; with the
 # accumulators forced into VGPR form the compiler crashes on them)
-AGPR_FORM_SOURCES = ("fa_bwd_d256_bf16.hip", "fa_bwd_d256_f16.hip")
+AGPR_FORM_SOURCES = ("fa_bwd_d256_bf16.hip", "fa_bwd_d256_f16.hip", "fa_bwd_cols256_bf16.hip",
+                     "fa_bwd_cols256_f16.hip")
 
 
 def hipcc() -> str:

@@ -452,11 +452,18 @@ size_t decode_ws_bytes(const fa_fwd_args* a, const fa::FwdParams& p) {
     return decode_part_rows(a, p) * (4 + (size_t)a->head_dim) * sizeof(float);
 }
 
+// head_cols of fa_fwd_cols / fa_bwd_cols: whole 16-byte chunks of 16-bit
+// columns, of a head dim that runs at the compiled one `D` (64, 128 or 256)
+bool cols_ok(int32_t cols, int32_t D, int32_t dtype, const void* bias, float dropout_p) {
+    return dtype != FA_DTYPE_F32 && !bias && !(dropout_p > 0.f) && D >= 64 && cols % 8 == 0 && cols > D / 2 && cols <= D;
+}
+
 // fa_fwd; with a workspace of fa_fwd_workspace_size bytes, the few-row path
-// where decode_plan takes it
-int32_t fwd_run(const fa_fwd_args* a, void* ws, size_t ws_bytes, bool allow_split, void* stream) {
+// where decode_plan takes it; cols: 0, or the columns that exist
+int32_t fwd_run(const fa_fwd_args* a, int32_t cols, void* ws, size_t ws_bytes, bool allow_split, void* stream) {
     int32_t st = fa_fwd_check(a);
     if (st) return st;
+    if (cols != 0 && !cols_ok(cols, a->head_dim, a->dtype, a->bias, a->dropout_p)) return FA_ERR_HEAD_DIM;
     if ((int64_t)a->batch * a->num_heads * a->seqlen_q == 0) return FA_OK;
     fa::FwdParams p{};
     if (allow_split && decode_plan(a, p) && p.dec_splits > 1) {
@@ -464,6 +471,7 @@ int32_t fwd_run(const fa_fwd_args* a, void* ws, size_t ws_bytes, bool allow_spli
         p.dec_stat = (float*)ws;
         p.dec_part = p.dec_stat + decode_part_rows(a, p) * 4;
     }
+    p.head_cols = cols < a->head_dim ? cols : 0;
     p.q = a->q;
     p.k = a->k;
     p.v = a->v;
@@ -530,7 +538,7 @@ int32_t fwd_run(const fa_fwd_args* a, void* ws, size_t ws_bytes, bool allow_spli
 
 extern "C" {
 
-int32_t fa_fwd(const fa_fwd_args* a, void* stream) { return fwd_run(a, nullptr, 0, false, stream); }
+int32_t fa_fwd(const fa_fwd_args* a, void* stream) { return fwd_run(a, 0, nullptr, 0, false, stream); }
 
 size_t fa_fwd_workspace_size(const fa_fwd_args* a) {
     if (!a) return 0;
@@ -543,7 +551,12 @@ size_t fa_fwd_workspace_size(const fa_fwd_args* a) {
 }
 
 int32_t fa_fwd_ws(const fa_fwd_args* a, void* workspace, size_t ws_bytes, void* stream) {
-    return fwd_run(a, workspace, ws_bytes, true, stream);
+    return fwd_run(a, 0, workspace, ws_bytes, true, stream);
+}
+
+int32_t fa_fwd_cols(const fa_fwd_args* a, int32_t head_cols, void* workspace, size_t ws_bytes, void* stream) {
+    if (head_cols <= 0) return FA_ERR_HEAD_DIM;
+    return fwd_run(a, head_cols, workspace, ws_bytes, true, stream);
 }
 
 size_t fa_bwd_workspace_size(const fa_bwd_args* a) {
@@ -594,16 +607,19 @@ namespace {
 
 // fa_bwd_stage; `side` allows the whole backward (stage -1) to write the zero
 // tails of a causal bias gradient on the library's side stream
-int32_t bwd_run(const fa_bwd_args* a, void* workspace, size_t ws_bytes, int32_t stage, void* stream, bool side) {
+int32_t bwd_run(const fa_bwd_args* a, int32_t cols, void* workspace, size_t ws_bytes, int32_t stage, void* stream,
+                bool side) {
     if (stage < -1 || stage > 3) return FA_ERR_SHAPE;
     int32_t st = fa_bwd_check(a, ws_bytes);
     if (st) return st;
+    if (cols != 0 && !cols_ok(cols, a->head_dim, a->dtype, a->bias, a->dropout_p)) return FA_ERR_HEAD_DIM;
     const size_t need = fa_bwd_workspace_size(a);
     if (need > 0 && (!workspace || !aligned16(workspace))) return FA_ERR_WORKSPACE;
     if ((int64_t)a->batch * a->num_heads * a->seqlen_q == 0 &&
         (int64_t)a->batch * a->num_heads_kv * a->seqlen_k == 0)
         return FA_OK;
     fa::BwdParams p{};
+    p.head_cols = cols < a->head_dim ? cols : 0;
     p.q = a->q;
     p.k = a->k;
     p.v = a->v;
@@ -781,11 +797,16 @@ int32_t bwd_run(const fa_bwd_args* a, void* workspace, size_t ws_bytes, int32_t 
 extern "C" {
 
 int32_t fa_bwd_stage(const fa_bwd_args* a, void* workspace, size_t ws_bytes, int32_t stage, void* stream) {
-    return bwd_run(a, workspace, ws_bytes, stage, stream, true);
+    return bwd_run(a, 0, workspace, ws_bytes, stage, stream, true);
 }
 
 int32_t fa_bwd(const fa_bwd_args* a, void* workspace, size_t ws_bytes, void* stream) {
-    return bwd_run(a, workspace, ws_bytes, -1, stream, true);
+    return bwd_run(a, 0, workspace, ws_bytes, -1, stream, true);
+}
+
+int32_t fa_bwd_cols(const fa_bwd_args* a, int32_t head_cols, void* workspace, size_t ws_bytes, void* stream) {
+    if (head_cols <= 0) return FA_ERR_HEAD_DIM;
+    return bwd_run(a, head_cols, workspace, ws_bytes, -1, stream, true);
 }
 
 int32_t fa_bwd_static(const fa_bwd_args* a, void* stream) {
@@ -800,7 +821,7 @@ int32_t fa_bwd_static(const fa_bwd_args* a, void* stream) {
     void* ws = static_scratch((hipStream_t)stream);
     if (!ws) return FA_ERR_LAUNCH;
     // one stream only: no library stream or event is created on this path
-    return bwd_run(a, ws, FA_BWD_STATIC_SCRATCH_BYTES, -1, stream, false);
+    return bwd_run(a, 0, ws, FA_BWD_STATIC_SCRATCH_BYTES, -1, stream, false);
 }
 
 int32_t fa_dropout_mask(uint64_t seed, uint64_t offset, int32_t B, int32_t H, int32_t Sq, int32_t Sk,

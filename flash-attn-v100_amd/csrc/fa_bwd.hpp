@@ -42,10 +42,16 @@ namespace fa {
 // padding rows (Sq <= i < sq_pad) get delta = 0 and LSE * log2(e) = +inf, so
 // a query tile that reads them gets P = 0 without a range check; so do rows
 // whose saved LSE is -inf.
+// (lanes per row: its 16-byte chunks rounded up to a power of two)
 template <typename T, int D>
-__global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
+struct DeltaRow {
+    static constexpr int CHUNKS = D * (int)sizeof(T) / 16;
+    static constexpr int LPR = CHUNKS <= 4 ? 4 : CHUNKS <= 8 ? 8 : CHUNKS <= 16 ? 16 : 32;
+};
+template <typename T, int D, typename P = BwdParams>
+__global__ __launch_bounds__(256) void delta_kernel(const P p) {
     constexpr int EPC = 16 / sizeof(T);
-    constexpr int LPR = D / EPC;        // lanes per row
+    constexpr int LPR = DeltaRow<T, D>::LPR;  // lanes per row
     constexpr int RPB = 256 / LPR;      // rows per block
     const int tid = threadIdx.x;
     const int64_t row = (int64_t)blockIdx.x * RPB + tid / LPR;
@@ -59,7 +65,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const BwdParams p) {
         i = (int)(bi % p.sq_pad);
         b = (int)(bi / p.sq_pad);
     }
-    if (row < nrows && i < p.Sq) {
+    if (row < nrows && i < p.Sq && part * EPC < ncols<D>(p)) {
         const T* orow = (const T*)p.o + b * p.o_sb + (int64_t)i * p.o_ss + h * p.o_sh + part * EPC;
         const T* drow = (const T*)p.dout + b * p.do_sb + (int64_t)i * p.do_ss + h * p.do_sh + part * EPC;
         const uint4 ov = *reinterpret_cast<const uint4*>(orow);
@@ -121,7 +127,7 @@ struct DkdvCfg {
     // Q / dO row stride: odd multiple of 16 bytes (conflict-free ds_read_b128
     // row reads) whose 4 consecutive rows of a ds_read_b64_tr_b16 do not overlap
     // in the 256-byte bank window
-    static constexpr int RW = D + (F32 ? 4 : (D == 64 ? 8 : 24));
+    static constexpr int RW = D + (F32 ? 4 : (D == 64 || D == 96 ? 8 : 24));
     static constexpr int QTILE = BQ * RW;
     // Q (waves 0-1) and dO (waves 2-3) tiles are copied global -> LDS directly
     using Rows = DmaRowGroups<T, BQ, D, RW, NW / 2>;
@@ -144,9 +150,9 @@ struct DkdvCfg {
 // (128 registers) do not fit the 512 registers of a lane, and spilled them
 // (about 1.1 KiB of scratch a lane); the halves recompute S and dP, 1.5x the
 // products of one launch, with nothing spilled.
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int DA = D, int DOFF = 0>
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int DA = D, int DOFF = 0, typename P = BwdParams>
 __global__ __launch_bounds__(256, ((std::is_void<TB>::value || D <= 64) && !(Elem<T>::kF32 && D == 128) && D <= 128 ? 2 : 1)) void dkdv_kernel(
-    const BwdParams p, const int n_ktiles) {
+    const P p, const int n_ktiles) {
     using C = DkdvCfg<T, D>;
     static_assert(DA % 32 == 0 && DOFF % 32 == 0 && DOFF + DA <= D, "a range of whole 32-column blocks");
     constexpr bool BIAS = !std::is_void<TB>::value;
@@ -180,7 +186,7 @@ __global__ __launch_bounds__(256, ((std::is_void<TB>::value || D <= 64) && !(Ele
 #pragma unroll
         for (int i = 0; i < KR; ++i) {
             const int d0 = C::F32 ? hi * (D / 2) + 4 * i : 16 * i + 8 * hi;
-            const bool ok = kj < p.Sk;
+            const bool ok = kj < p.Sk && d0 < ncols<D>(p);
             kreg[i] = ok ? *reinterpret_cast<const uint4*>(krow + d0) : make_uint4(0u, 0u, 0u, 0u);
             vreg[i] = ok ? *reinterpret_cast<const uint4*>(vrow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
@@ -213,7 +219,7 @@ __global__ __launch_bounds__(256, ((std::is_void<TB>::value || D <= 64) && !(Ele
     // same values), so a tile copy is branch-free and can sit between MFMAs
     const bool copy_q = w < C::NW / 2;
     typename C::Rows rows;
-    rows.init(copy_q ? p.q_ss : p.do_ss, lane, w % (C::NW / 2));
+    rows.init(copy_q ? p.q_ss : p.do_ss, lane, w % (C::NW / 2), ncols<D>(p));
     static_assert(BQ == 64, "one dword per lane for each of LSE and delta");
     auto buf = [&](int s) -> char* { return smem + s * C::BUF_BYTES; };
     auto tile_head = [&](int it) { return hk * p.group + it / nq; };
@@ -522,7 +528,7 @@ __global__ __launch_bounds__(256, ((std::is_void<TB>::value || D <= 64) && !(Ele
             const int cidx = lane + 64 * i;
             const int row = cidx / CPR, col = cidx % CPR;
             const int key = kw0 + row;
-            if (key < p.Sk)
+            if (key < p.Sk && DOFF + col * EPC < ncols<D>(p))
                 *reinterpret_cast<uint4*>(gbase + (int64_t)key * gss + DOFF + col * EPC) =
                     *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
         }
@@ -564,7 +570,9 @@ struct DkdvPPCfg {
     static constexpr int NT = 64 * NW;
     static constexpr int BK = 32 * NW;               // keys per workgroup
     static constexpr int BQ = 64;                    // queries per tile: two 32-query sub-steps
-    static constexpr int RW = D + 24;                // Q / dO row stride, as in dkdv_kernel
+    // Q / dO row stride, as in dkdv_kernel at D = 128 (D = 96 keeps it, and with
+    // it the copy schedule; its further padding chunks read nothing)
+    static constexpr int RW = D + (D == 96 ? 56 : 24);
     static constexpr int QALLOC = BQ * RW * (int)sizeof(T);
     // per slot: Q rows, dO rows, then LSE * log2 e [BQ] and delta [BQ] as floats
     static constexpr int SLOT_BYTES = 2 * QALLOC + 2 * BQ * 4;
@@ -584,10 +592,10 @@ struct DkdvPPCfg {
     static_assert(SLOT_BYTES % 16 == 0, "16-byte aligned slots");
 };
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const BwdParams p, const int n_ktiles) {
+template <typename T, int D, bool CAUSAL, typename P = BwdParams>
+__global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const P p, const int n_ktiles) {
     using C = DkdvPPCfg<T, D>;
-    static_assert(!Elem<T>::kF32 && D == 128, "16-bit inputs, D = 128");
+    static_assert(!Elem<T>::kF32 && (D == 128 || D == 96), "16-bit inputs");
     constexpr int BQ = C::BQ, RW = C::RW;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
 
@@ -612,8 +620,9 @@ __global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const BwdParams p, cons
 #pragma unroll
         for (int i = 0; i < KR; ++i) {
             const int d0 = 16 * i + 8 * hi;
-            kreg[i] = ok ? *reinterpret_cast<const uint4*>(krow + d0) : make_uint4(0u, 0u, 0u, 0u);
-            vreg[i] = ok ? *reinterpret_cast<const uint4*>(vrow + d0) : make_uint4(0u, 0u, 0u, 0u);
+            const bool okd = ok && d0 < ncols<D>(p);
+            kreg[i] = okd ? *reinterpret_cast<const uint4*>(krow + d0) : make_uint4(0u, 0u, 0u, 0u);
+            vreg[i] = okd ? *reinterpret_cast<const uint4*>(vrow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
         // -V: the dP products start from delta and give delta - dP (as dkdv_kernel)
 #pragma unroll
@@ -679,7 +688,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const BwdParams p, cons
         for (int n = 0; n < 3; ++n) {
             const int cidx = 64 * (8 * n + 4 * hf + w4) + lane;
             const int row = cidx / C::CW, col = cidx % C::CW;
-            coff[hf][n] = col < D / C::EPC ? (row * (int)css + col * C::EPC) * (int)sizeof(T) : kOffNowhere;
+            coff[hf][n] = col < ncols<D>(p) / C::EPC ? (row * (int)css + col * C::EPC) * (int)sizeof(T) : kOffNowhere;
         }
     // The copy position: the current tile's sources and ranges (rows and the
     // workspace row) and LDS slot, advanced one tile at a time by additions:
@@ -979,7 +988,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const BwdParams p, cons
             const int cidx = lane + 64 * i;
             const int row = cidx / CPR, col = cidx % CPR;
             const int key = kw0 + row;
-            if (key < p.Sk)
+            if (key < p.Sk && col * EPC < ncols<D>(p))
                 *reinterpret_cast<uint4*>(gbase + (int64_t)key * gss + col * EPC) =
                     *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
         }
@@ -1010,7 +1019,7 @@ struct Dkdv8Cfg {
     static constexpr int NT = 64 * NW;
     static constexpr int BK = 128;                  // keys per workgroup
     static constexpr int BQ = 64;                   // queries per tile
-    static constexpr int RW = D + (D == 64 ? 8 : 24);  // Q / dO rows, as in DkdvCfg
+    static constexpr int RW = D + (D == 64 || D == 96 ? 8 : 24);  // Q / dO rows, as in DkdvCfg
     static constexpr int KVW = D + 8;               // K / V rows (conflict-free b128 row reads)
     static constexpr int QALLOC = BQ * RW * (int)sizeof(T);
     static constexpr int BUF_BYTES = 2 * QALLOC + 2 * BQ * 4;
@@ -1027,8 +1036,8 @@ struct Dkdv8Cfg {
 };
 
 // (bid, nblocks: this workgroup among the dK/dV ones; smem: Dkdv8Cfg::SMEM_BYTES of LDS)
-template <typename T, int D, bool CAUSAL, typename TB>
-__device__ FA_INLINE inline void dkdv8_body(const BwdParams& p, const int n_ktiles, const int bid, const int nblocks,
+template <typename T, int D, bool CAUSAL, typename TB, typename P>
+__device__ FA_INLINE inline void dkdv8_body(const P& p, const int n_ktiles, const int bid, const int nblocks,
                                            char* smem) {
     using C = Dkdv8Cfg<T, D>;
     static_assert(!Elem<T>::kF32, "16-bit inputs");
@@ -1053,10 +1062,10 @@ __device__ FA_INLINE inline void dkdv8_body(const BwdParams& p, const int n_ktil
     char* bufs = smem + 2 * C::KV_BYTES;
     {  // K and V rows of the 128 keys (rows past Sk land as zeros)
         typename C::KV kd;
-        kd.init(p.k_ss, lane, w);
+        kd.init(p.k_ss, lane, w, ncols<D>(p));
         kd.load_untracked((const T*)p.k + b * p.k_sb + (int64_t)k0 * p.k_ss + hk * p.k_sh, p.k_ss, p.Sk - k0, Ks, lane);
         typename C::KV vd;
-        vd.init(p.v_ss, lane, w);
+        vd.init(p.v_ss, lane, w, ncols<D>(p));
         vd.load_untracked((const T*)p.v + b * p.v_sb + (int64_t)k0 * p.v_ss + hk * p.v_sh, p.v_ss, p.Sk - k0, Vs, lane);
     }
 
@@ -1075,7 +1084,7 @@ __device__ FA_INLINE inline void dkdv8_body(const BwdParams& p, const int n_ktil
 
     const bool copy_q = w < 4;
     typename C::Rows rows;
-    rows.init(copy_q ? p.q_ss : p.do_ss, lane, w & 3);
+    rows.init(copy_q ? p.q_ss : p.do_ss, lane, w & 3, ncols<D>(p));
     auto buf = [&](int s) -> char* { return bufs + s * C::BUF_BYTES; };
     auto tile_head = [&](int it) { return hk * p.group + it / nq; };
     auto tile_q0 = [&](int it) { return (qt_end - 1 - it % nq) * BQ; };
@@ -1330,7 +1339,7 @@ __device__ FA_INLINE inline void dkdv8_body(const BwdParams& p, const int n_ktil
                 const int cidx = lane + 64 * i;
                 const int row = cidx / CPR, col = cidx % CPR;
                 const int key = kw0 + row;
-                if (key < p.Sk)
+                if (key < p.Sk && col * EPC < ncols<D>(p))
                     *reinterpret_cast<uint4*>(gbase + (int64_t)key * gss + col * EPC) =
                         *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
             }
@@ -1338,8 +1347,8 @@ __device__ FA_INLINE inline void dkdv8_body(const BwdParams& p, const int n_ktil
     }
 }
 
-template <typename T, int D, bool CAUSAL, typename TB>
-__global__ __launch_bounds__(512, 1) void dkdv8_kernel(const BwdParams p, const int n_ktiles) {
+template <typename T, int D, bool CAUSAL, typename TB, typename P = BwdParams>
+__global__ __launch_bounds__(512, 1) void dkdv8_kernel(const P p, const int n_ktiles) {
     __shared__ __attribute__((aligned(16))) char smem[Dkdv8Cfg<T, D>::SMEM_BYTES];
     dkdv8_body<T, D, CAUSAL, TB>(p, n_ktiles, (int)blockIdx.x, (int)gridDim.x, smem);
 }
@@ -1356,7 +1365,7 @@ struct DqCfg {
     static constexpr int BN = 32 * NSUB;          // keys per tile
     // K / V row stride: conflict-free ds_read_b128 row reads and (16-bit)
     // ds_read_b64_tr_b16 reads of K^T, as for the dK/dV tiles
-    static constexpr int KW = D + (F32 ? 4 : (D == 64 ? 8 : 24));
+    static constexpr int KW = D + (F32 ? 4 : (D == 64 || D == 96 ? 8 : 24));
     // K (waves 0-1) and V (waves 2-3) tiles are copied global -> LDS directly
     using Rows = DmaRowGroups<T, BN, D, KW, NW / 2>;
     static constexpr int KALLOC = BN * KW * (int)sizeof(T);
@@ -1373,8 +1382,8 @@ struct DqCfg {
 // queries, group sp walking key tiles sp, sp + KS, ... through its own LDS
 // buffers; their dQ partials are summed through LDS at the end (small grids).
 // (bid, nblocks: this workgroup among the dQ ones; smem: KS * DqCfg::SMEM_BYTES of LDS)
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS>
-__device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles, const int bid, const int nblocks,
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, typename P>
+__device__ FA_INLINE inline void dq_body(const P& p, const int n_qtiles, const int bid, const int nblocks,
                                         char* smem) {
     using C = DqCfg<T, D>;
     constexpr bool BIAS = !std::is_void<TB>::value;
@@ -1406,7 +1415,7 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
 #pragma unroll
         for (int i = 0; i < QR; ++i) {
             const int d0 = C::F32 ? hi * (D / 2) + 4 * i : 16 * i + 8 * hi;
-            const bool ok = qi < p.Sq;
+            const bool ok = qi < p.Sq && d0 < ncols<D>(p);
             qreg[i] = ok ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0u, 0u, 0u, 0u);
             doreg[i] = ok ? *reinterpret_cast<const uint4*>(drow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
@@ -1414,8 +1423,9 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
             if (own_delta) {
 #pragma unroll
                 for (int i = 0; i < QR; ++i)
-                    oreg[i] = qi < p.Sq ? *reinterpret_cast<const uint4*>(orow + 16 * i + 8 * hi)
-                                        : make_uint4(0u, 0u, 0u, 0u);
+                    oreg[i] = qi < p.Sq && 16 * i + 8 * hi < ncols<D>(p)
+                                  ? *reinterpret_cast<const uint4*>(orow + 16 * i + 8 * hi)
+                                  : make_uint4(0u, 0u, 0u, 0u);
             }
         }
     }
@@ -1454,7 +1464,7 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
     const T* vbase = (const T*)p.v + b * p.v_sb + hk * p.v_sh;
     const bool copy_k = w < C::NW / 2;
     typename C::Rows rows;
-    rows.init(copy_k ? p.k_ss : p.v_ss, lane, w % (C::NW / 2));
+    rows.init(copy_k ? p.k_ss : p.v_ss, lane, w % (C::NW / 2), ncols<D>(p));
     auto buf = [&](int s) -> char* { return smem + sp * C::SMEM_BYTES + s * C::BUF_BYTES; };
     auto issue = [&](int j, int s) FA_INLINE {
         const int k0 = (j * KS + sp) * BN;
@@ -1485,6 +1495,7 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
             // chunks (chunk sums, then a pairwise tree), so both give the same
             // bits; the rows go to the workspace for the dK/dV pass, which runs
             // after this one.  Rows past Sq: delta = 0, LSE * log2 e = +inf.
+            constexpr int QR2 = QR <= 2 ? 2 : QR <= 4 ? 4 : QR <= 8 ? 8 : 16;  // chunk slots of the tree
             float cs[QR];
 #pragma unroll
             for (int i = 0; i < QR; ++i) {
@@ -1495,9 +1506,10 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
                 cs[i] = acc;
             }
 #pragma unroll
-            for (int st = QR / 2; st > 0; st >>= 1)
+            for (int st = QR2 / 2; st > 0; st >>= 1)
 #pragma unroll
-                for (int i = 0; i < st; ++i) cs[i] = cs[i] + cs[i + st];
+                for (int i = 0; i < st; ++i)
+                    if (i + st < QR) cs[i] = cs[i] + cs[i + st];
             del = pair_sum(cs[0]);
             lse2 = lse_in == -INFINITY ? INFINITY : lse_in * kLog2e;
             if (sp == 0 && hi == 0) {
@@ -1747,15 +1759,15 @@ __device__ FA_INLINE inline void dq_body(const BwdParams& p, const int n_qtiles,
             const int cidx = lane + 64 * i;
             const int row = cidx / CPR, col = cidx % CPR;
             const int q = qw0 + row;
-            if (q < p.Sq)
+            if (q < p.Sq && col * EPC < ncols<D>(p))
                 *reinterpret_cast<uint4*>(gbase + (int64_t)q * p.dq_ss + col * EPC) =
                     *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
         }
     }
 }
 
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS>
-__global__ __launch_bounds__(256 * KS, (KS == 1 ? DqCfg<T, D>::MIN_BLOCKS : 1)) void dq_kernel(const BwdParams p,
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, typename P = BwdParams>
+__global__ __launch_bounds__(256 * KS, (KS == 1 ? DqCfg<T, D>::MIN_BLOCKS : 1)) void dq_kernel(const P p,
                                                                                            const int n_qtiles) {
     __shared__ __attribute__((aligned(16))) char smem[DqCfg<T, D>::SMEM_BYTES * KS];
     dq_body<T, D, CAUSAL, DROPOUT, TB, KS>(p, n_qtiles, (int)blockIdx.x, (int)gridDim.x, smem);
@@ -1778,8 +1790,8 @@ struct BwdSmallCfg {
     static_assert(SMEM_BYTES <= 160 * 1024, "LDS of one CU");
 };
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void bwd_small_kernel(const BwdParams p, const int n_ktiles, const int n_kv,
+template <typename T, int D, bool CAUSAL, typename P = BwdParams>
+__global__ __launch_bounds__(512, 1) void bwd_small_kernel(const P p, const int n_ktiles, const int n_kv,
                                                           const int n_qtiles, const int n_q) {
     __shared__ __attribute__((aligned(16))) char smem[BwdSmallCfg<T, D>::SMEM_BYTES];
     // workgroups 2 i and 2 i + 1 take the i-th dK/dV and dQ ones while both
@@ -1829,7 +1841,8 @@ struct DqPPCfg {
     static constexpr int NT = 64 * NW;
     static constexpr int BM = 32 * NW;               // queries per workgroup
     static constexpr int BN = 64;                    // keys per tile
-    static constexpr int KW = D + 24;                // K / V row stride, as in dq_kernel
+    // K / V row stride, as in dq_kernel at D = 128 (D = 96 too: banks)
+    static constexpr int KW = D + (D == 96 ? 56 : 24);
     static constexpr int KALLOC = BN * KW * (int)sizeof(T);
     static constexpr int SLOT_BYTES = 2 * KALLOC;    // K rows, V rows
     static constexpr int NSLOT = 4;
@@ -1844,10 +1857,10 @@ struct DqPPCfg {
     static_assert(NW * 32 * OW * (int)sizeof(T) <= SMEM_BYTES, "output staging");
 };
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
+template <typename T, int D, bool CAUSAL, typename P = BwdParams>
+__global__ __launch_bounds__(512, 1) void dq_pp_kernel(const P p) {
     using C = DqPPCfg<T, D>;
-    static_assert(!Elem<T>::kF32 && D == 128, "16-bit inputs, D = 128");
+    static_assert(!Elem<T>::kF32 && (D == 128 || D == 96), "16-bit inputs");
     constexpr int BN = C::BN, KW = C::KW, NSLOT = C::NSLOT;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
 
@@ -1874,10 +1887,14 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
     constexpr int QR = D / 16;
     const bool own_delta = p.dq_delta != 0;
     const int qrows = min(p.Sq - q0, C::BM);  // >= 1: q0 < Sq
-    auto rows_rsrc = [&](const void* base, int64_t ss) FA_INLINE {
-        return slice_buffer((const T*)base + (int64_t)q0 * ss, ((qrows - 1) * (int)ss + D) * (int)sizeof(T));
-    };
     const int rrow = 32 * blk + l32;  // this lane's row in the block
+    auto rows_rsrc = [&](const void* base, int64_t ss) FA_INLINE {
+        return slice_buffer((const T*)base + (int64_t)q0 * ss, ((qrows - 1) * (int)ss + ncols<D>(p)) * (int)sizeof(T));
+    };
+    // a chunk of columns that do not exist is sent out of range
+    auto row_off = [&](int64_t ss, int d0) FA_INLINE {
+        return d0 < ncols<D>(p) ? (rrow * (int)ss + d0) * (int)sizeof(T) : kOffNowhere;
+    };
     uint4 qreg[QR], doreg[QR], oreg[QR];
     {
         const __amdgpu_buffer_rsrc_t rq = rows_rsrc((const T*)p.q + b * p.q_sb + h * p.q_sh, p.q_ss);
@@ -1886,16 +1903,16 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
         for (int i = 0; i < QR; ++i) {
             const int d0 = 16 * i + 8 * hi;
             qreg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                    rq, (rrow * (int)p.q_ss + d0) * (int)sizeof(T), 0, 0));
+                                                    rq, row_off(p.q_ss, d0), 0, 0));
             doreg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                     rd, (rrow * (int)p.do_ss + d0) * (int)sizeof(T), 0, 0));
+                                                     rd, row_off(p.do_ss, d0), 0, 0));
         }
         if (own_delta) {
             const __amdgpu_buffer_rsrc_t ro = rows_rsrc((const T*)p.o + b * p.o_sb + h * p.o_sh, p.o_ss);
 #pragma unroll
             for (int i = 0; i < QR; ++i)
                 oreg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        ro, (rrow * (int)p.o_ss + 16 * i + 8 * hi) * (int)sizeof(T), 0, 0));
+                                                        ro, row_off(p.o_ss, 16 * i + 8 * hi), 0, 0));
         }
     }
     // the workspace rows hold sq_pad (Sq rounded up to 128) entries; the last
@@ -1947,7 +1964,7 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
         const int cidx = 64 * (w4 + 4 * t) + lane;
         const int row = cidx / C::CW, col = cidx % C::CW;
         // padding chunks of an LDS row read nothing (out of the buffer's range)
-        coff[t] = col < D / C::EPC ? (row * (int)css + col * C::EPC) * (int)sizeof(T) : kOffNowhere;
+        coff[t] = col < ncols<D>(p) / C::EPC ? (row * (int)css + col * C::EPC) * (int)sizeof(T) : kOffNowhere;
     }
     auto slot = [&](int r) FA_INLINE -> char* { return smem + (r & (NSLOT - 1)) * C::SLOT_BYTES; };
     static_assert(NSLOT == 4, "slot index by mask");
@@ -2103,6 +2120,7 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
         // delta = rowsum(dO * O) as dq_kernel computes it (16-byte chunk sums,
         // then a pairwise tree, then the lane pair), written to the workspace
         // with LSE * log2 e; rows past Sq: delta = 0, LSE * log2 e = +inf
+        constexpr int QR2 = 8;  // chunk slots of the tree (QR = 6 or 8)
         float cs[QR];
 #pragma unroll
         for (int i = 0; i < QR; ++i) {
@@ -2113,9 +2131,10 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
             cs[i] = acc;
         }
 #pragma unroll
-        for (int st = QR / 2; st > 0; st >>= 1)
+        for (int st = QR2 / 2; st > 0; st >>= 1)
 #pragma unroll
-            for (int i = 0; i < st; ++i) cs[i] = cs[i] + cs[i + st];
+            for (int i = 0; i < st; ++i)
+                if (i + st < QR) cs[i] = cs[i] + cs[i + st];
         del = pair_sum(cs[0]);
         const float lse_in = qi < p.Sq ? lse_raw : -INFINITY;
         lse2 = lse_in == -INFINITY ? INFINITY : lse_in * kLog2e;
@@ -2206,7 +2225,7 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const BwdParams p) {
         const int cidx = lane + 64 * i;
         const int row = cidx / CPR, col = cidx % CPR;
         const int q = qw0 + row;
-        if (q < p.Sq)
+        if (q < p.Sq && col * EPC < ncols<D>(p))
             *reinterpret_cast<uint4*>(gbase + (int64_t)q * p.dq_ss + col * EPC) =
                 *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
     }
@@ -2442,14 +2461,14 @@ inline bool dq_pp_runs(const BwdParams& p) {
 }
 
 // Whether the whole backward runs as the delta pre-pass plus bwd_small_kernel
-// (16-bit inputs, D = 64 or 128, no bias or dropout): where dK/dV would run
+// (16-bit inputs, D = 64 to 128, no bias or dropout): where dK/dV would run
 // dkdv8_kernel on fewer workgroups than CUs and dQ the key-split dq_kernel,
 // and either both kinds of workgroups fit the CUs at once or the mask makes
 // their tile chains uneven (non-causal chains of one length on more workgroups
 // than CUs gain nothing from sharing them and would pay the pre-pass).
 template <typename T, int D, bool CAUSAL>
 inline bool bwd_small_runs(const BwdParams& p) {
-    if constexpr (!Elem<T>::kF32 && (D == 64 || D == 128) && 2 * DqCfg<T, D>::SMEM_BYTES <= 160 * 1024) {
+    if constexpr (!Elem<T>::kF32 && (D == 64 || D == 96 || D == 128) && 2 * DqCfg<T, D>::SMEM_BYTES <= 160 * 1024) {
         const int64_t nq = (int64_t)((p.Sq + DqCfg<T, D>::BM - 1) / DqCfg<T, D>::BM) * p.H * p.B;
         const int64_t nkv = (int64_t)((p.Sk + Dkdv8Cfg<T, D>::BK - 1) / Dkdv8Cfg<T, D>::BK) * p.Hkv * p.B;
         return dkdv8_runs<T, D, CAUSAL, 0, void>(p) && nq > 0 && nq < 256 && p.Sk > DqCfg<T, D>::BN &&
@@ -2458,18 +2477,18 @@ inline bool bwd_small_runs(const BwdParams& p) {
     return false;
 }
 
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB>
-hipError_t launch_bwd_t(const BwdParams& p0, int stage, hipStream_t s) {
-    if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 64 || D == 128)) {
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, typename P>
+hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
+    if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 64 || D == 96 || D == 128)) {
         if (stage < 0 && bwd_small_runs<T, D, CAUSAL>(p0)) {
-            hipError_t e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB>(p0, 0, s);  // delta rows
+            hipError_t e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(p0, 0, s);  // delta rows
             if (e != hipSuccess) return e;
-            BwdParams pr = p0;
+            P pr = p0;
             pr.dq_delta = 0;  // dQ reads the delta rows
             const int nk = (p0.Sk + Dkdv8Cfg<T, D>::BK - 1) / Dkdv8Cfg<T, D>::BK;
             const int nq = (p0.Sq + DqCfg<T, D>::BM - 1) / DqCfg<T, D>::BM;
             const int n_kv = nk * p0.Hkv * p0.B, n_q = nq * p0.H * p0.B;
-            hipLaunchKernelGGL((bwd_small_kernel<T, D, CAUSAL>), dim3((unsigned)(n_kv + n_q)), dim3(512), 0, s, pr, nk,
+            hipLaunchKernelGGL((bwd_small_kernel<T, D, CAUSAL, P>), dim3((unsigned)(n_kv + n_q)), dim3(512), 0, s, pr, nk,
                                n_kv, nq, n_q);
             return hipGetLastError();
         }
@@ -2482,42 +2501,41 @@ hipError_t launch_bwd_t(const BwdParams& p0, int stage, hipStream_t s) {
     if (stage == 3 || (stage < 0 && !ds_pass)) {
         hipError_t e;
         if constexpr (Elem<T>::kF32) {
-            e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB>(p0, 0, s);
-            if (e == hipSuccess) e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB>(p0, 2, s);
+            e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(p0, 0, s);
+            if (e == hipSuccess) e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(p0, 2, s);
         } else {
-            BwdParams pf = p0;
+            P pf = p0;
             pf.dq_delta = 1;
-            e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB>(pf, 2, s);
+            e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(pf, 2, s);
         }
         if (e != hipSuccess || stage == 3) return e;
-        return launch_bwd_t<T, D, CAUSAL, DROPOUT, TB>(p0, 1, s);
+        return launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(p0, 1, s);
     }
-    const BwdParams& p = p0;
+    const P& p = p0;
     if (stage < 0 || stage == 0) {
-        constexpr int EPC = 16 / sizeof(T);
-        constexpr int RPB = 256 / (D / EPC);
+        constexpr int RPB = 256 / DeltaRow<T, D>::LPR;
         const int64_t nrows = (int64_t)p.B * p.sq_pad * p.H;
         const int64_t nb = (nrows + RPB - 1) / RPB;
-        if (nb > 0) hipLaunchKernelGGL((delta_kernel<T, D>), dim3((unsigned)nb), dim3(256), 0, s, p);
+        if (nb > 0) hipLaunchKernelGGL((delta_kernel<T, D, P>), dim3((unsigned)nb), dim3(256), 0, s, p);
     }
     if (stage < 0 || stage == 1) {
         using C = DkdvCfg<T, D>;
         const int nk = (p.Sk + C::BK - 1) / C::BK;
         const int64_t nb = (int64_t)nk * p.Hkv * p.B;
         bool done = false;
-        if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && D == 128) {
+        if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
             if (dkdv_pp_runs(p)) {
                 using CP = DkdvPPCfg<T, D>;
                 const int nk2 = (p.Sk + CP::BK - 1) / CP::BK;
                 const int64_t nb2 = (int64_t)nk2 * p.Hkv * p.B;
-                hipLaunchKernelGGL((dkdv_pp_kernel<T, D, CAUSAL>), dim3((unsigned)nb2), dim3(CP::NT), 0, s, p, nk2);
+                hipLaunchKernelGGL((dkdv_pp_kernel<T, D, CAUSAL, P>), dim3((unsigned)nb2), dim3(CP::NT), 0, s, p, nk2);
                 done = true;
             }
         }
         if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && D >= 64 && D <= 128) {
             static_assert(Dkdv8Cfg<T, D>::BK == C::BK, "same key blocks");
             if (!done && dkdv8_runs<T, D, CAUSAL, DROPOUT, TB>(p)) {
-                hipLaunchKernelGGL((dkdv8_kernel<T, D, CAUSAL, TB>), dim3((unsigned)nb), dim3(Dkdv8Cfg<T, D>::NT), 0, s, p,
+                hipLaunchKernelGGL((dkdv8_kernel<T, D, CAUSAL, TB, P>), dim3((unsigned)nb), dim3(Dkdv8Cfg<T, D>::NT), 0, s, p,
                                    nk);
                 done = true;
             }
@@ -2525,14 +2543,14 @@ hipError_t launch_bwd_t(const BwdParams& p0, int stage, hipStream_t s) {
         if constexpr (D == 256) {
             // two launches of 128 dK / dV columns each (see dkdv_kernel)
             if (!done && nb > 0) {
-                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, 128, 0>), dim3((unsigned)nb), dim3(C::NT), 0, s,
+                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, 128, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0, s,
                                    p, nk);
-                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, 128, 128>), dim3((unsigned)nb), dim3(C::NT), 0,
+                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, 128, 128, P>), dim3((unsigned)nb), dim3(C::NT), 0,
                                    s, p, nk);
             }
         } else {
             if (!done && nb > 0)
-                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nk);
+                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, D, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nk);
         }
     }
     if (stage < 0 || stage == 2) {
@@ -2554,11 +2572,11 @@ hipError_t launch_bwd_t(const BwdParams& p0, int stage, hipStream_t s) {
                 done = true;
             }
         }
-        if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && D == 128) {
+        if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
             if (!done && dq_pp_runs(p)) {
                 using CP = DqPPCfg<T, D>;
                 const int64_t nb2 = (int64_t)((p.Sq + CP::BM - 1) / CP::BM) * p.H * p.B;
-                hipLaunchKernelGGL((dq_pp_kernel<T, D, CAUSAL>), dim3((unsigned)nb2), dim3(CP::NT), 0, s, p);
+                hipLaunchKernelGGL((dq_pp_kernel<T, D, CAUSAL, P>), dim3((unsigned)nb2), dim3(CP::NT), 0, s, p);
                 done = true;
             }
         }
@@ -2566,19 +2584,28 @@ hipError_t launch_bwd_t(const BwdParams& p0, int stage, hipStream_t s) {
         // the workgroup (as the forward does) where two splits' tiles fit the LDS
         if constexpr (2 * C::SMEM_BYTES <= 160 * 1024) {
             if (!done && nb > 0 && nb < 256 && p.Sk > C::BN) {
-                hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 2>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s,
+                hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 2, P>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s,
                                    p, nq);
                 done = true;
             }
         }
         if (!done && nb > 0)
-            hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
+            hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
     }
     return hipGetLastError();
 }
 
+// head dims between the compiled ones (p.head_cols; fa_cols.hpp)
+template <typename T>
+hipError_t launch_bwd_cols(const BwdParams& p, int D, bool causal, int stage, hipStream_t s);
+template <typename T>
+hipError_t launch_bwd_cols256(const BwdParams& p, bool causal, int stage, hipStream_t s);
+
 template <typename T, typename TB>
 hipError_t launch_bwd_dispatch(const BwdParams& p, int D, bool causal, bool dropout, int stage, hipStream_t s) {
+    if constexpr (!Elem<T>::kF32 && std::is_void<TB>::value) {
+        if (p.head_cols > 0) return launch_bwd_cols<T>(p, D, causal, stage, s);
+    }
     // dropout mode: 0 none, 1 Philox mask regenerated, 2 the forward's keep bits read
     const int mode = !dropout ? 0 : (p.kb != nullptr ? 2 : 1);
 #define FA_BWD_MODES(DD, CC)                                                \
@@ -2605,6 +2632,7 @@ hipError_t launch_bwd_dispatch(const BwdParams& p, int D, bool causal, bool drop
 template <typename T>
 hipError_t launch_bwd_d256(const BwdParams& p, bool causal, bool dropout, int stage, hipStream_t s) {
     static_assert(!Elem<T>::kF32, "16-bit inputs");
+    if (p.head_cols > 0) return launch_bwd_cols256<T>(p, causal, stage, s);
     const int mode = !dropout ? 0 : (p.kb != nullptr ? 2 : 1);
 #define FA_BWD_MODES(CC)                                                    \
     switch (mode) {                                                         \

@@ -505,14 +505,16 @@ struct DmaTile {
 
     // wave_id must be wave-uniform (readfirstlane): it selects the LDS
     // destination, which the hardware takes from a scalar register (M0).
-    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id) {
+    // cols: the columns that exist (at most D, whole 16-byte chunks); the
+    // others land as zeros
+    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int cols = D) {
         wave = wave_id;
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int c = 64 * (wave + NW * t) + lane;
             const int row = c / CW, col = c % CW;
             // padding chunks of an LDS row read nothing (out of the buffer's range)
-            off[t] = col < CD ? (row * (int)row_stride + col * EPC) * (int)sizeof(T) : kOffNowhere;
+            off[t] = col < cols / EPC ? (row * (int)row_stride + col * EPC) * (int)sizeof(T) : kOffNowhere;
         }
     }
     __device__ FA_INLINE inline void load(const T* base, int64_t row_stride, int nvalid, T* lds, int lane) const {
@@ -618,14 +620,14 @@ struct DmaRowGroups {
     int rowl;  // this lane's row within the group (KR for idle lanes)
     int wave;
 
-    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id) {
+    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int cols = D) {
         wave = wave_id;
         rowl = lane < KR * CW ? lane / CW : KR;
         // padding chunks read nothing: an offset past the range stays past it
         // (below 2^32) after the group's row step is added (tiles span < 2^31
         // bytes)
         const int col = lane % CW;
-        off = col < CD ? ((lane / CW) * (int)row_stride + col * EPC) * (int)sizeof(T) : kOffNowhere;
+        off = col < cols / EPC ? ((lane / CW) * (int)row_stride + col * EPC) * (int)sizeof(T) : kOffNowhere;
     }
     __device__ FA_INLINE inline void load(const T* base, int64_t row_stride, int nvalid, T* lds) const {
         const __amdgpu_buffer_rsrc_t rs = row_buffer<T, D, R>(base, row_stride, nvalid);

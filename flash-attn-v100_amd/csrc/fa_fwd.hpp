@@ -44,7 +44,7 @@ struct FwdCfg {
     static constexpr int KW = D + (F32 ? 4 : 8);  // K row stride (elements)
     // V rows; 16-bit types read V^T fragments with ds_read_b64_tr_b16, whose
     // four rows per lane group fall in distinct banks at this stride
-    static constexpr int VW = F32 ? D + 8 : D + (D == 64 ? 8 : 24);
+    static constexpr int VW = F32 ? D + 8 : D + (D == 64 || D == 96 ? 8 : 24);
     static constexpr int KTILE = BN * KW;
     static constexpr int VTILE = BN * VW;
     static constexpr int OW = D + (F32 ? 4 : 8);  // output staging row stride
@@ -65,8 +65,8 @@ struct FwdCfg {
 // region: 16-byte copies along the rows, where per-lane loads (one query row
 // per lane) touch 32 rows per instruction.  The LDS of one such workgroup
 // holds the K/V tiles and the 8 bias regions.
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, int QG = 1>
-__global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 : 1) void fwd_kernel(const FwdParams p) {
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, int QG = 1, typename P = FwdParams>
+__global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 : 1) void fwd_kernel(const P p) {
     using C = FwdCfg<T, D>;
     constexpr bool BIAS = !std::is_void<TB>::value;
     using BT = typename std::conditional<BIAS, TB, T>::type;
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         for (int i = 0; i < QR; ++i) {
             // bf16/f16: d = 16i + 8hi .. +7 ; f32: d = hi*D/2 + 4i .. +3
             const int d0 = C::F32 ? hi * (D / 2) + 4 * i : 16 * i + 8 * hi;
-            qreg[i] = qi < p.Sq ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0u, 0u, 0u, 0u);
+            qreg[i] = qi < p.Sq && d0 < ncols<D>(p) ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
     }
     // no wait here: the Q loads stay in flight while the first tile copies
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     // pipeline below issues them unconditionally; such tiles are never used.
     const int wv = __builtin_amdgcn_readfirstlane(QG > 1 ? wg : w);
     DmaTile<T, BN, D, KW, C::NW * QG> kdma;
-    kdma.init(p.k_ss, lane, wv);
+    kdma.init(p.k_ss, lane, wv, ncols<D>(p));
     // 16-bit tiles: copies the compiler does not track, which it would
     // otherwise make the next LDS read wait for (sync_tiles waits for them)
     auto dma_k = [&](int j, int slot) {
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
             kdma.load_untracked(kbase + (int64_t)k0 * p.k_ss, p.k_ss, p.Sk - k0, Ks0 + slot * C::KTILE, lane);
     };
     DmaTile<T, BN, D, VW, C::NW * QG> vst;
-    vst.init(p.v_ss, lane, wv);
+    vst.init(p.v_ss, lane, wv, ncols<D>(p));
     auto load_v = [&](int j, int slot) {
         const int k0 = key0(j);
         if constexpr (C::F32)
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
             const int cidx = lane + 64 * i;
             const int row = cidx / CPR, col = cidx % CPR;
             const int q = qw0 + row;
-            if (q < p.Sq)
+            if (q < p.Sq && col * EPC < ncols<D>(p))
                 *reinterpret_cast<uint4*>(obase + (int64_t)q * p.o_ss + col * EPC) =
                     *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
         }
@@ -574,7 +574,7 @@ struct FwdPPCfg {
     static constexpr int NB = BN / 32;            // 32-key blocks per tile
     static constexpr int NSLOT = 4;               // K / V tile slots
     static constexpr int KW = D + 8;              // K row stride (elements)
-    static constexpr int VW = D + (D == 64 ? 8 : 24);
+    static constexpr int VW = D + (D == 64 || D == 96 ? 8 : 24);
     static constexpr int KTILE = BN * KW;
     static constexpr int VTILE = BN * VW;
     static constexpr int OW = D + 8;              // output staging row stride
@@ -583,8 +583,8 @@ struct FwdPPCfg {
     static_assert(SMEM_ELEMS * 2 <= 160 * 1024, "LDS of one CU");
 };
 
-template <typename T, int D, bool CAUSAL, bool FIT>
-__global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const FwdParams p) {
+template <typename T, int D, bool CAUSAL, bool FIT, typename P = FwdParams>
+__global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const P p) {
     using C = FwdPPCfg<T, D>;
     static_assert(!Elem<T>::kF32, "16-bit inputs");
     constexpr int BN = C::BN, NB = C::NB, KW = C::KW, VW = C::VW, NSLOT = C::NSLOT;
@@ -624,9 +624,9 @@ __global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const FwdParams p) {
         // both groups have finished.  Tiles past Sk read nothing and land as
         // zeros.  At most 63 copy instructions are in flight (the vmcnt range).
         DmaTile<T, BN, D, KW, 1> kd;
-        kd.init(p.k_ss, lane, 0);
+        kd.init(p.k_ss, lane, 0, ncols<D>(p));
         DmaTile<T, BN, D, VW, 1> vd;
-        vd.init(p.v_ss, lane, 0);
+        vd.init(p.v_ss, lane, 0, ncols<D>(p));
         constexpr int NKI = decltype(kd)::NI, NVI = decltype(vd)::NI;
         static_assert(2 * NKI + NVI <= 63, "vmcnt range");
         // keys past the workgroup's last tile are never read: copies of tiles
@@ -667,7 +667,8 @@ __global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const FwdParams p) {
         const T* qrow = (const T*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh;
 #pragma unroll
         for (int i = 0; i < QR; ++i)
-            qreg[i] = qi < p.Sq ? *reinterpret_cast<const uint4*>(qrow + 16 * i + 8 * hi) : make_uint4(0u, 0u, 0u, 0u);
+            qreg[i] = qi < p.Sq && 16 * i + 8 * hi < ncols<D>(p) ? *reinterpret_cast<const uint4*>(qrow + 16 * i + 8 * hi)
+                                                               : make_uint4(0u, 0u, 0u, 0u);
     }
 
     f32x16 o[D / 32];
@@ -680,9 +681,9 @@ __global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const FwdParams p) {
 
     // prologue copies: the 8 compute waves (in the loop: the copy wave)
     DmaTile<T, BN, D, KW, C::NW> kdma;
-    kdma.init(p.k_ss, lane, w);
+    kdma.init(p.k_ss, lane, w, ncols<D>(p));
     DmaTile<T, BN, D, VW, C::NW> vdma;
-    vdma.init(p.v_ss, lane, w);
+    vdma.init(p.v_ss, lane, w, ncols<D>(p));
     auto dma_k = [&](int j) FA_INLINE {
         if (j < n_tiles)
             kdma.load(kbase + (int64_t)(j * BN) * p.k_ss, p.k_ss, p.Sk - j * BN, Ks0 + (j % NSLOT) * C::KTILE, lane);
@@ -874,7 +875,7 @@ __global__ __launch_bounds__(576, 1) void fwd_pp_kernel(const FwdParams p) {
         const int cidx = lane + 64 * i;
         const int row = cidx / CPR, col = cidx % CPR;
         const int q = qw0 + row;
-        if (q < p.Sq)
+        if (q < p.Sq && col * EPC < ncols<D>(p))
             *reinterpret_cast<uint4*>(obase + (int64_t)q * p.o_ss + col * EPC) =
                 *reinterpret_cast<const uint4*>(Os + row * OW + col * EPC);
     }
@@ -901,20 +902,20 @@ inline bool fwd_pp_wanted(const FwdParams& p, bool causal) {
     return n >= 256 && (!causal || (p.Sq >= 3072 && n >= 512));
 }
 
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB>
-hipError_t launch_fwd_t(const FwdParams& p, hipStream_t s) {
-    if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && D == 128) {
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, typename P>
+hipError_t launch_fwd_t(const P& p, hipStream_t s) {
+    if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
         if (fwd_pp_wanted(p, CAUSAL)) {
             using CP = FwdPPCfg<T, D>;
-            FwdParams q = p;
+            P q = p;
             q.n_qtiles = (p.Sq + CP::BM - 1) / CP::BM;
             const int64_t nblocks = (int64_t)q.n_qtiles * p.H * p.B;
             // causal rows differ in length, so a small last slice group runs
             // its long rows alone: (2, 3072, 32) 173.0 -> 155.7 us with FIT
-            if constexpr (CAUSAL) {
+            if constexpr (CAUSAL && std::is_same<P, FwdParams>::value) {
                 if (host_group_uneven(32, q.n_qtiles, (int)nblocks)) return launch_fwd_pp_fit<T>(q, nblocks, s);
             }
-            hipLaunchKernelGGL((fwd_pp_kernel<T, D, CAUSAL, false>), dim3((unsigned)nblocks), dim3(CP::NT), 0, s, q);
+            hipLaunchKernelGGL((fwd_pp_kernel<T, D, CAUSAL, false, P>), dim3((unsigned)nblocks), dim3(CP::NT), 0, s, q);
             return hipGetLastError();
         }
     }
@@ -924,16 +925,16 @@ hipError_t launch_fwd_t(const FwdParams& p, hipStream_t s) {
     // 16-byte chunks
     if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && !std::is_void<TB>::value) {
         if constexpr (!Elem<TB>::kF32) {
-            FwdParams q = p;
+            P q = p;
             q.n_qtiles = (p.Sq + 2 * C::BM - 1) / (2 * C::BM);
             const int64_t nb2 = (int64_t)q.n_qtiles * p.H * p.B;
             if (nb2 >= 256 && p.Sk % 8 == 0) {
-                hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, 0, TB, 1, 2>), dim3((unsigned)nb2), dim3(C::NT * 2), 0, s, q);
+                hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, 0, TB, 1, 2, P>), dim3((unsigned)nb2), dim3(C::NT * 2), 0, s, q);
                 return hipGetLastError();
             }
         }
     }
-    FwdParams q = p;
+    P q = p;
     q.n_qtiles = (p.Sq + C::BM - 1) / C::BM;
     const int64_t nblocks = (int64_t)q.n_qtiles * p.H * p.B;
     if (nblocks <= 0) return hipSuccess;
@@ -945,23 +946,27 @@ hipError_t launch_fwd_t(const FwdParams& p, hipStream_t s) {
     // (D = 256: one workgroup's tiles take most of the LDS, no split)
     if constexpr (D <= 128) {
         if (nblocks < n_cu && p.Sk > C::BN) {
-            hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, KS_SMALL>), dim3((unsigned)nblocks),
+            hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, KS_SMALL, 1, P>), dim3((unsigned)nblocks),
                                dim3(C::NT * KS_SMALL), 0, s, q);
             return hipGetLastError();
         }
     }
-    hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, 1>), dim3((unsigned)nblocks), dim3(C::NT), 0, s, q);
+    hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, 1, 1, P>), dim3((unsigned)nblocks), dim3(C::NT), 0, s, q);
     return hipGetLastError();
 }
 
 // The few-row forward (fa_fwd_decode.hpp, instantiated in fa_fwd_decode.hip)
 template <typename T>
 hipError_t launch_fwd_decode(const FwdParams& p, int D, bool causal, hipStream_t s);
+// head dims between the compiled ones (p.head_cols; fa_cols.hpp)
+template <typename T>
+hipError_t launch_fwd_cols(const FwdParams& p, int D, bool causal, hipStream_t s);
 
 template <typename T, typename TB>
 hipError_t launch_fwd_dispatch(const FwdParams& p, int D, bool causal, bool dropout, hipStream_t s) {
     if constexpr (!Elem<T>::kF32 && std::is_void<TB>::value) {
         if (p.dec_splits > 0) return launch_fwd_decode<T>(p, D, causal, s);
+        if (p.head_cols > 0) return launch_fwd_cols<T>(p, D, causal, s);
     }
     // dropout mode: 0 none, 1 Philox mask, 2 Philox mask also written as keep bits
     const int mode = !dropout ? 0 : (p.kb != nullptr ? 2 : 1);
@@ -990,6 +995,7 @@ hipError_t launch_fwd_dispatch(const FwdParams& p, int D, bool causal, bool drop
 template <typename T>
 hipError_t launch_fwd_d256(const FwdParams& p, bool causal, bool dropout, hipStream_t s) {
     static_assert(!Elem<T>::kF32, "16-bit inputs");
+    if (p.head_cols > 0) return launch_fwd_cols<T>(p, 256, causal, s);
     const int mode = !dropout ? 0 : (p.kb != nullptr ? 2 : 1);
 #define FA_FWD_MODES(CC)                                                    \
     switch (mode) {                                                         \

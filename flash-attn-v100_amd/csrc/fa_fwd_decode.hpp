@@ -36,15 +36,15 @@ struct FwdDecCfg {
     static constexpr int BN = 64;                 // keys per tile
     static constexpr int NB = BN / 32;
     static constexpr int KW = D + 8;              // LDS row strides as in FwdCfg
-    static constexpr int VW = D + (D == 64 ? 8 : 24);
+    static constexpr int VW = D + (D == 64 || D == 96 ? 8 : 24);
     static constexpr int KTILE = BN * KW;
     static constexpr int VTILE = BN * VW;
     static constexpr int REGION = KTILE + VTILE;  // elements of a wave's LDS region
     static_assert((D / 32) * 16 * 64 * 4 <= REGION * 2, "a wave's O part fits its region");
 };
 
-template <typename T, int D, bool CAUSAL>
-__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const FwdParams p) {
+template <typename T, int D, bool CAUSAL, typename P = FwdParams>
+__global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const P p) {
     using C = FwdDecCfg<T, D>;
     static_assert(!Elem<T>::kF32, "16-bit inputs");
     constexpr int BN = C::BN, NB = C::NB, KW = C::KW, VW = C::VW;
@@ -83,9 +83,9 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
     T* Ks = smem + w * C::REGION;
     T* Vs = Ks + C::KTILE;
     DmaTile<T, BN, D, KW, 1> kd;
-    kd.init(p.k_ss, lane, 0);
+    kd.init(p.k_ss, lane, 0, ncols<D>(p));
     DmaTile<T, BN, D, VW, 1> vd;
-    vd.init(p.v_ss, lane, 0);
+    vd.init(p.v_ss, lane, 0, ncols<D>(p));
     constexpr int NKI = decltype(kd)::NI, NVI = decltype(vd)::NI;
     static_assert(NKI + NVI <= 63, "vmcnt range");
     // tiles past the split's end read nothing (empty range) but are issued, so
@@ -103,7 +103,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
         const T* qrow = (const T*)p.q + b * p.q_sb + (int64_t)i * p.q_ss + h * p.q_sh;
 #pragma unroll
         for (int kk = 0; kk < QR; ++kk)
-            qreg[kk] = live ? *reinterpret_cast<const uint4*>(qrow + 16 * kk + 8 * hi) : make_uint4(0u, 0u, 0u, 0u);
+            qreg[kk] = live && 16 * kk + 8 * hi < ncols<D>(p) ? *reinterpret_cast<const uint4*>(qrow + 16 * kk + 8 * hi)
+                                                                 : make_uint4(0u, 0u, 0u, 0u);
     }
     // the Q loads have completed before the copies below are issued: the
     // compiler's own waits for them then never wait for a copy
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
                 s16x4 v4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v4[e] = Elem<T>::pack1(om[4 * q4 + e] * inv);
-                *reinterpret_cast<s16x4*>(ob + 8 * q4) = v4;
+                if (32 * n + 8 * q4 < ncols<D>(p)) *reinterpret_cast<s16x4*>(ob + 8 * q4) = v4;
             }
         }
     }
@@ -276,8 +277,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
 
 // The splits' parts of every row, rescaled to their common maximum and
 // normalised: one thread per 4 columns of a row (D / 4 threads share a row).
-template <typename T, int D>
-__global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p, const int n_rows) {
+template <typename T, int D, typename P = FwdParams>
+__global__ __launch_bounds__(256) void fwd_combine_kernel(const P p, const int n_rows) {
     constexpr int TPR = D / 4;  // threads per row
     const int gid = (int)blockIdx.x * 256 + (int)threadIdx.x;
     const int r = gid / TPR, col = (gid % TPR) * 4;
@@ -310,26 +311,33 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const FwdParams p, con
     s16x4 v4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v4[e] = Elem<T>::pack1(acc[e] * inv);
-    *reinterpret_cast<s16x4*>((T*)p.o + b * p.o_sb + (int64_t)i * p.o_ss + h * p.o_sh + col) = v4;
+    if (col < ncols<D>(p)) *reinterpret_cast<s16x4*>((T*)p.o + b * p.o_sb + (int64_t)i * p.o_ss + h * p.o_sh + col) = v4;
 }
 
-template <typename T, int D>
-hipError_t launch_fwd_decode_t(const FwdParams& p, bool causal, hipStream_t s) {
+template <typename T, int D, typename P>
+hipError_t launch_fwd_decode_t(const P& p, bool causal, hipStream_t s) {
     const int64_t nb = (int64_t)p.B * p.Hkv * p.dec_rt * p.dec_splits;
     if (causal)
-        hipLaunchKernelGGL((fwd_decode_kernel<T, D, true>), dim3((unsigned)nb), dim3(256), 0, s, p);
+        hipLaunchKernelGGL((fwd_decode_kernel<T, D, true, P>), dim3((unsigned)nb), dim3(256), 0, s, p);
     else
-        hipLaunchKernelGGL((fwd_decode_kernel<T, D, false>), dim3((unsigned)nb), dim3(256), 0, s, p);
+        hipLaunchKernelGGL((fwd_decode_kernel<T, D, false, P>), dim3((unsigned)nb), dim3(256), 0, s, p);
     if (p.dec_splits > 1) {
         const int n_rows = p.B * p.H * p.Sq;
         const int64_t nt = (int64_t)n_rows * (D / 4);
-        hipLaunchKernelGGL((fwd_combine_kernel<T, D>), dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, p, n_rows);
+        hipLaunchKernelGGL((fwd_combine_kernel<T, D, P>), dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, p, n_rows);
     }
     return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_fwd_decode(const FwdParams& p, int D, bool causal, hipStream_t s) {
+    if (p.head_cols > 0) {
+        FwdParamsCols pc;
+        static_cast<FwdParams&>(pc) = p;
+        if (D == 64) return launch_fwd_decode_t<T, 64>(pc, causal, s);
+        if (D == 128 && p.head_cols <= 96) return launch_fwd_decode_t<T, 96>(pc, causal, s);
+        return D == 128 ? launch_fwd_decode_t<T, 128>(pc, causal, s) : hipErrorInvalidValue;
+    }
     switch (D) {
         case 32: return launch_fwd_decode_t<T, 32>(p, causal, s);
         case 64: return launch_fwd_decode_t<T, 64>(p, causal, s);

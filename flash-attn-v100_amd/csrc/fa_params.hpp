@@ -44,6 +44,9 @@ struct FwdParams {
     int dec_splits, dec_rt;
     float* dec_stat;
     float* dec_part;
+    // columns of q, k, v and o that exist (a multiple of 8; 0: all D): a head
+    // dim between the compiled ones (FwdParamsCols)
+    int head_cols;
 };
 
 struct BwdParams {
@@ -97,11 +100,27 @@ struct BwdParams {
     // aligned and Sk * dbias_es is a multiple of 16
     int dq_from_ds;
     int ds_span;  // readable bytes of one (batch, head) dS slice (dq_from_ds)
+    int head_cols;  // as in FwdParams
     // 1 (set by the launcher, 16-bit inputs): the dQ pass runs first and
     // computes LSE * log2 e and delta of its query rows itself, writing the
     // workspace rows the dK/dV pass then reads (no delta pre-pass)
     int dq_delta;
 };
+
+// The same parameters for the instantiations that read and write the columns
+// [0, head_cols) of a row only: the others are zeros in LDS and registers (they
+// add nothing to a product) and are never stored.  ncols<D>(p) is the constant
+// D for the plain parameters, whose kernels compile as if it were not there.
+struct FwdParamsCols : FwdParams {};
+struct BwdParamsCols : BwdParams {};
+template <int D>
+__host__ __device__ constexpr int ncols(const FwdParams&) { return D; }
+template <int D>
+__host__ __device__ constexpr int ncols(const BwdParams&) { return D; }
+template <int D>
+__host__ __device__ constexpr int ncols(const FwdParamsCols& p) { return p.head_cols; }
+template <int D>
+__host__ __device__ constexpr int ncols(const BwdParamsCols& p) { return p.head_cols; }
 
 // Sum of per-(batch, head) dBias slices over broadcast dimensions:
 // out[bo][ho][i][j] = sum of part[b][h][i][j] over b (sum_b) / h (sum_h);

@@ -74,7 +74,8 @@ class BwdArgs(ctypes.Structure):
 
 
 EXPORTS = (
-    "fa_abi_version", "fa_strerror", "fa_fwd_check", "fa_fwd", "fa_fwd_workspace_size", "fa_fwd_ws",
+    "fa_abi_version", "fa_strerror", "fa_fwd_check", "fa_fwd", "fa_fwd_workspace_size", "fa_fwd_ws", "fa_fwd_cols",
+    "fa_bwd_cols",
     "fa_bwd_workspace_size",
     "fa_bwd_check", "fa_bwd", "fa_bwd_stage", "fa_bwd_static", "fa_dropout_mask", "fa_rand",
 )
@@ -112,6 +113,10 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fa_fwd_workspace_size.argtypes = [P(FwdArgs)]
     lib.fa_fwd_ws.restype = ctypes.c_int32
     lib.fa_fwd_ws.argtypes = [P(FwdArgs), ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    lib.fa_fwd_cols.restype = ctypes.c_int32
+    lib.fa_fwd_cols.argtypes = [P(FwdArgs), ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    lib.fa_bwd_cols.restype = ctypes.c_int32
+    lib.fa_bwd_cols.argtypes = [P(BwdArgs), ctypes.c_int32, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
     lib.fa_bwd_workspace_size.restype = ctypes.c_size_t
     lib.fa_bwd_workspace_size.argtypes = [P(BwdArgs)]
     lib.fa_bwd_check.restype = ctypes.c_int32
@@ -177,6 +182,13 @@ def padded_head_dim(d: int, dtype: Optional[torch.dtype] = None, bias: bool = Fa
     if d <= WIDE_HEAD_DIM and dtype in (torch.float16, torch.bfloat16) and not bias:
         return WIDE_HEAD_DIM
     return 0
+
+
+def _cols_run(d: int, dp: int, dtype: torch.dtype, bias, dropout_p: float) -> bool:
+    """Whether a head dim of ``d`` runs at the compiled one ``dp`` on the
+    tensors as they are (``fa_fwd_cols`` / ``fa_bwd_cols``: whole 16-byte chunks
+    of 16-bit columns, no bias or dropout) instead of on zero-padded copies."""
+    return dp >= 64 and d != dp and d % 8 == 0 and dtype != torch.float32 and bias is None and not dropout_p > 0
 
 
 def _pad_d(t: torch.Tensor, dp: int) -> torch.Tensor:
@@ -300,8 +312,9 @@ def _check_keep_bits(bits: torch.Tensor, B, H, Sq, Sk, device):
 
 
 def fwd_args(q, k, v, o, lse, max_vals, causal, scale, dropout_p, seed, offset, bias=None,
-             keep_bits=None) -> FwdArgs:
+             keep_bits=None, head_dim=None) -> FwdArgs:
     B, Sq, H, D = q.shape
+    D = head_dim or D
     return FwdArgs(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
         max_vals.data_ptr() if max_vals is not None else None,
@@ -331,7 +344,8 @@ def fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: 
     lib = load()
     D = q.shape[-1]
     dp = padded_head_dim(D, q.dtype, bias is not None) or D  # no kernel: the library rejects it
-    q, k, v = (prepare(_pad_d(t, dp)) for t in (q, k, v))
+    cols = _cols_run(D, dp, q.dtype, bias, dropout_p)
+    q, k, v = (prepare(t if cols else _pad_d(t, dp)) for t in (q, k, v))
     pb = _as_prepared(bias, q, k)
     B, Sq, H, _ = q.shape
     o = torch.empty_like(q, memory_format=torch.contiguous_format)
@@ -339,16 +353,21 @@ def fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: 
     mx = torch.empty((B, H, Sq), device=q.device, dtype=torch.float32) if want_max else None
     if keep_bits is not None:
         _check_keep_bits(keep_bits, B, H, Sq, k.shape[1], q.device)
-    a = fwd_args(q, k, v, o, lse, mx, causal, scale, dropout_p, seed, offset, pb, keep_bits)
+    a = fwd_args(q, k, v, o, lse, mx, causal, scale, dropout_p, seed, offset, pb, keep_bits, dp)
     ws_bytes = lib.fa_fwd_workspace_size(ctypes.byref(a))
     ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
-    _check("fa_fwd_ws", lib.fa_fwd_ws(ctypes.byref(a), ws.data_ptr() if ws_bytes else None, ws_bytes, _stream(q)))
+    wp = ws.data_ptr() if ws_bytes else None
+    if cols:
+        _check("fa_fwd_cols", lib.fa_fwd_cols(ctypes.byref(a), D, wp, ws_bytes, _stream(q)))
+    else:
+        _check("fa_fwd_ws", lib.fa_fwd_ws(ctypes.byref(a), wp, ws_bytes, _stream(q)))
     return _unpad_d(o, D), lse, mx
 
 
 def bwd_args(q, k, v, o, do, lse, dq, dk, dv, causal, scale, dropout_p, seed, offset,
-             bias=None, dbias=None, keep_bits=None) -> BwdArgs:
+             bias=None, dbias=None, keep_bits=None, head_dim=None) -> BwdArgs:
     B, Sq, H, D = q.shape
+    D = head_dim or D
     return BwdArgs(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(),
         dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
@@ -381,7 +400,8 @@ def bwd(q, k, v, o, do, lse, causal: bool, scale: float, dropout_p: float = 0.0,
     lib = load()
     D = q.shape[-1]
     dp = padded_head_dim(D, q.dtype, bias is not None) or D
-    q, k, v, o, do = (prepare(_pad_d(t, dp)) for t in (q, k, v, o, do))
+    cols = _cols_run(D, dp, q.dtype, bias, dropout_p)
+    q, k, v, o, do = (prepare(t if cols else _pad_d(t, dp)) for t in (q, k, v, o, do))
     pb = _as_prepared(bias, q, k)
     if want_dbias and pb is None:
         raise ValueError("want_dbias needs a bias")
@@ -407,10 +427,14 @@ def bwd(q, k, v, o, do, lse, causal: bool, scale: float, dropout_p: float = 0.0,
             dbias = torch.empty((Bo, Ho, Sq, -(-Sk // 4) * 4), device=q.device, dtype=gdt)[..., :Sk]
     if keep_bits is not None:
         _check_keep_bits(keep_bits, q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.device)
-    a = bwd_args(q, k, v, o, do, lse, dq, dk, dv, causal, scale, dropout_p, seed, offset, pb, dbias, keep_bits)
+    a = bwd_args(q, k, v, o, do, lse, dq, dk, dv, causal, scale, dropout_p, seed, offset, pb, dbias, keep_bits,
+                 dp)
     ws_bytes = lib.fa_bwd_workspace_size(ctypes.byref(a))
     ws = torch.empty(max(int(ws_bytes), 256), device=q.device, dtype=torch.uint8)
-    _check("fa_bwd", lib.fa_bwd(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(q)))
+    if cols:
+        _check("fa_bwd_cols", lib.fa_bwd_cols(ctypes.byref(a), D, ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(q)))
+    else:
+        _check("fa_bwd", lib.fa_bwd(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(q)))
     dq, dk, dv = (_unpad_d(t, D) for t in (dq, dk, dv))
     if want_dbias:
         return dq, dk, dv, reduce_dbias(dbias, pb)

@@ -190,8 +190,8 @@ int32_t fa_fwd_check(const fa_fwd_args* args);
 int32_t fa_fwd(const fa_fwd_args* args, void* hip_stream);
 
 /* Bytes of device workspace fa_fwd_ws needs: for few query rows over many
- * keys (16-bit inputs, no causal mask, bias or dropout) the keys may be split
- * over several workgroups, whose float32 parts of every row go there; 0 where
+ * keys (16-bit inputs, no bias or dropout) the keys may be split over several
+ * workgroups, whose float32 parts of every row go there; 0 where
  * none is needed and on invalid arguments.  Host-only.  No reference
  * counterpart. */
 size_t fa_fwd_workspace_size(const fa_fwd_args* args);
@@ -201,6 +201,18 @@ size_t fa_fwd_workspace_size(const fa_fwd_args* args);
  * hip_stream has run): the same results, up to the order of the float32 sums
  * where the keys are split.  FA_ERR_WORKSPACE if it is missing or too small. */
 int32_t fa_fwd_ws(const fa_fwd_args* args, void* workspace, size_t workspace_bytes, void* hip_stream);
+
+/* fa_fwd_ws / fa_bwd for a head dim between the compiled ones, without padded
+ * copies: 16-bit inputs without bias or dropout.  head_dim is the compiled
+ * head dim it runs at (64, 128 or 256), head_cols the columns that exist, a
+ * multiple of 8 in (head_dim / 2, head_dim]: only those of q, k, v, o, dout are
+ * read and only those of o, dq, dk, dv written, through strides that meet the
+ * usual rules.  Same results as on zero-padded tensors.  FA_ERR_HEAD_DIM for
+ * anything else.  No reference counterpart (its tiles masked the columns). */
+int32_t fa_fwd_cols(const fa_fwd_args* args, int32_t head_cols, void* workspace, size_t workspace_bytes,
+                    void* hip_stream);
+int32_t fa_bwd_cols(const fa_bwd_args* args, int32_t head_cols, void* workspace, size_t workspace_bytes,
+                    void* hip_stream);
 
 /* Bytes of device workspace fa_bwd needs: B * H rows of 2 * sq_pad float32
  * (sq_pad = Sq rounded up to 128; LSE * log2 e then delta = rowsum(dO * O),
