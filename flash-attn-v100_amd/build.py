@@ -1,4 +1,5 @@
-"""Build the gfx950 kernel library ``flash_attention_v100/libfa_gfx950.so``.
+"""Build the gfx950 kernel library ``flash_attention_v100/libfa_gfx950.so`` and
+the CPython module of its per-call host path, ``flash_attention_v100/fa_host.so``.
 
 Compiles every translation unit in ``csrc/`` with hipcc for gfx950 (in
 parallel), then links one shared library exporting the C ABI of
@@ -21,6 +22,8 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "flash_attention_v100", "libfa_gfx950.so")
+HOST_SRC = os.path.join(CSRC, "fa_host.cpp")
+HOST_LIB = os.path.join(HERE, "flash_attention_v100", "fa_host.so")
 ARCH = "gfx950"
 
 _H, _A = ("bf16", "f16"), ("bf16", "f16", "f32")
@@ -94,11 +97,37 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_host() -> str:
+    """The CPython module of the per-call host path (host code only, against
+    the headers and libraries of the torch that imports it)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    tmp = HOST_LIB + ".tmp"
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           "-I", INCLUDE, "-isystem", sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include"]
+    for d in cpp_extension.include_paths():
+        cmd += ["-isystem", d]
+    cmd += ["-o", tmp, HOST_SRC]
+    for d in cpp_extension.library_paths():
+        cmd += ["-L", d]
+    cmd += ["-lc10", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {HOST_SRC}\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, HOST_LIB)
+    return HOST_LIB
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> str:
     os.makedirs(OBJDIR, exist_ok=True)
     jobs = jobs or min(len(SOURCES), max(1, os.cpu_count() or 1))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(build_host)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

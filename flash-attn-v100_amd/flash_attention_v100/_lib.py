@@ -1,23 +1,27 @@
-"""ctypes binding of the gfx950 kernel library (``libfa_gfx950.so``).
+"""Binding of the gfx950 kernel library (``libfa_gfx950.so``).
 
 The library exports the C ABI of ``include/fa_abi.h``.  This module mirrors its
-argument structs, loads it (after torch, so that both share torch's HIP
+argument structs (ctypes), loads it (after torch, so that both share torch's HIP
 runtime: the library's ``libamdhip64.so.7`` dependency resolves to the copy
-torch already loaded) and turns status codes into exceptions.  All memory is
-allocated here with torch; the library itself never allocates.
+torch already loaded) and turns status codes into exceptions.  :func:`fwd` and
+:func:`bwd` run the per-call host path in ``fa_host.so`` (``csrc/fa_host.cpp``).
+All memory is allocated with torch; the library itself never allocates.
 
-There is no fallback: if the library is missing or fails to load, every entry
-point raises :class:`FlashAttentionExtensionError`.
+There is no fallback: if either library is missing or fails to load, every
+entry point raises :class:`FlashAttentionExtensionError`.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional, Tuple
 
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libfa_gfx950.so")
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "fa_host.so")
 ABI_VERSION = 3
 HEAD_DIMS = (32, 64, 128)  # compiled into the kernels for every dtype, with or without a bias
 WIDE_HEAD_DIM = 256        # compiled for fp16 / bf16 inputs without a bias
@@ -138,6 +142,35 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         raise FlashAttentionExtensionError(f"{path} has ABI version {v}, expected {ABI_VERSION}")
     _lib = lib
     return lib
+
+
+_host_mod = None
+
+
+def _host():
+    """The module of the per-call host path, bound (once) to the library."""
+    global _host_mod
+    if _host_mod is not None:
+        return _host_mod
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise FlashAttentionExtensionError(
+            f"host module not found at {HOST_PATH}; build it with `python flash-attn-v100_amd/build.py`")
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("fa_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("fa_host", loader))
+        loader.exec_module(mod)
+    except ImportError as e:  # pragma: no cover - depends on the machine
+        raise FlashAttentionExtensionError(f"cannot load {HOST_PATH}: {e}") from e
+    mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
+        lib.fa_fwd_workspace_size, lib.fa_fwd_ws, lib.fa_fwd_cols, lib.fa_bwd_workspace_size, lib.fa_bwd,
+        lib.fa_bwd_cols)))
+    _host_mod = mod
+    return mod
+
+
+def _raw_stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def strerror(code: int) -> str:
@@ -341,27 +374,27 @@ def fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, scale: 
     :class:`PreparedBias`;
     ``keep_bits`` (from :func:`alloc_keep_bits`, with dropout) receives the
     keep mask applied."""
-    lib = load()
+    host = _host()
     D = q.shape[-1]
     dp = padded_head_dim(D, q.dtype, bias is not None) or D  # no kernel: the library rejects it
-    cols = _cols_run(D, dp, q.dtype, bias, dropout_p)
-    q, k, v = (prepare(t if cols else _pad_d(t, dp)) for t in (q, k, v))
+    cols = 0
+    if dp != D:
+        if _cols_run(D, dp, q.dtype, bias, dropout_p):
+            cols = D
+        else:
+            q, k, v = (_pad_d(t, dp) for t in (q, k, v))
     pb = _as_prepared(bias, q, k)
-    B, Sq, H, _ = q.shape
-    o = torch.empty_like(q, memory_format=torch.contiguous_format)
-    lse = torch.empty((B, H, Sq), device=q.device, dtype=torch.float32)
-    mx = torch.empty((B, H, Sq), device=q.device, dtype=torch.float32) if want_max else None
     if keep_bits is not None:
-        _check_keep_bits(keep_bits, B, H, Sq, k.shape[1], q.device)
-    a = fwd_args(q, k, v, o, lse, mx, causal, scale, dropout_p, seed, offset, pb, keep_bits, dp)
-    ws_bytes = lib.fa_fwd_workspace_size(ctypes.byref(a))
-    ws = torch.empty(ws_bytes, device=q.device, dtype=torch.uint8) if ws_bytes else None
-    wp = ws.data_ptr() if ws_bytes else None
-    if cols:
-        _check("fa_fwd_cols", lib.fa_fwd_cols(ctypes.byref(a), D, wp, ws_bytes, _stream(q)))
-    else:
-        _check("fa_fwd_ws", lib.fa_fwd_ws(ctypes.byref(a), wp, ws_bytes, _stream(q)))
-    return _unpad_d(o, D), lse, mx
+        _check_keep_bits(keep_bits, q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.device)
+    st, o, lse, mx = host.fwd(q, k, v, causal, scale, dropout_p, seed, offset,
+                              *_NO_BIAS if pb is None else (pb.tensor, tuple(pb.strides), pb.dtype_code),
+                              keep_bits, want_max, dp, cols, _raw_stream(q))
+    if st:
+        _check("fa_fwd", st)
+    return (o if cols else _unpad_d(o, D)), lse, mx
+
+
+_NO_BIAS = (None, None, 0)
 
 
 def bwd_args(q, k, v, o, do, lse, dq, dk, dv, causal, scale, dropout_p, seed, offset,
@@ -397,18 +430,18 @@ def bwd(q, k, v, o, do, lse, causal: bool, scale: float, dropout_p: float = 0.0,
     gradient in the caller's bias shape and dtype when ``want_dbias``.
     ``keep_bits``: the mask the forward wrote (same seed / offset), read
     instead of regenerating it."""
-    lib = load()
+    host = _host()
     D = q.shape[-1]
     dp = padded_head_dim(D, q.dtype, bias is not None) or D
-    cols = _cols_run(D, dp, q.dtype, bias, dropout_p)
-    q, k, v, o, do = (prepare(t if cols else _pad_d(t, dp)) for t in (q, k, v, o, do))
+    cols = 0
+    if dp != D:
+        if _cols_run(D, dp, q.dtype, bias, dropout_p):
+            cols = D
+        else:
+            q, k, v, o, do = (_pad_d(t, dp) for t in (q, k, v, o, do))
     pb = _as_prepared(bias, q, k)
     if want_dbias and pb is None:
         raise ValueError("want_dbias needs a bias")
-    lse = lse.contiguous()
-    dq = torch.empty_like(q, memory_format=torch.contiguous_format)
-    dk = torch.empty_like(k, memory_format=torch.contiguous_format)
-    dv = torch.empty_like(v, memory_format=torch.contiguous_format)
     dbias = None
     if want_dbias:
         B, Sq, H, _ = q.shape
@@ -427,15 +460,16 @@ def bwd(q, k, v, o, do, lse, causal: bool, scale: float, dropout_p: float = 0.0,
             dbias = torch.empty((Bo, Ho, Sq, -(-Sk // 4) * 4), device=q.device, dtype=gdt)[..., :Sk]
     if keep_bits is not None:
         _check_keep_bits(keep_bits, q.shape[0], q.shape[2], q.shape[1], k.shape[1], q.device)
-    a = bwd_args(q, k, v, o, do, lse, dq, dk, dv, causal, scale, dropout_p, seed, offset, pb, dbias, keep_bits,
-                 dp)
-    ws_bytes = lib.fa_bwd_workspace_size(ctypes.byref(a))
-    ws = torch.empty(max(int(ws_bytes), 256), device=q.device, dtype=torch.uint8)
-    if cols:
-        _check("fa_bwd_cols", lib.fa_bwd_cols(ctypes.byref(a), D, ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(q)))
-    else:
-        _check("fa_bwd", lib.fa_bwd(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(), _stream(q)))
-    dq, dk, dv = (_unpad_d(t, D) for t in (dq, dk, dv))
+    st, dq, dk, dv = host.bwd(q, k, v, o, do, lse, causal, scale, dropout_p, seed, offset,
+                              *_NO_BIAS if pb is None else (pb.tensor, tuple(pb.strides), pb.dtype_code),
+                              keep_bits,
+                              *_NO_BIAS if dbias is None else (dbias, tuple(_dbias_strides(dbias)),
+                                                               DTYPE_CODES[dbias.dtype]),
+                              dp, cols, _raw_stream(q))
+    if st:
+        _check("fa_bwd", st)
+    if dp != D and not cols:
+        dq, dk, dv = (_unpad_d(t, D) for t in (dq, dk, dv))
     if want_dbias:
         return dq, dk, dv, reduce_dbias(dbias, pb)
     return dq, dk, dv

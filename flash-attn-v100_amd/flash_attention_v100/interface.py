@@ -49,7 +49,7 @@ def validate_inputs_enhanced(q, k, v, scale=None, bias=None, dropout_p=0.0):
     """Metadata checks with the reference's error types and messages
     (``utils.py:31-160``); returns (q, k, v, scale) with the default
     ``scale = head_dim ** -0.5`` (``utils.py:148-153``)."""
-    if not all(isinstance(t, torch.Tensor) for t in (q, k, v)):
+    if not (isinstance(q, torch.Tensor) and isinstance(k, torch.Tensor) and isinstance(v, torch.Tensor)):
         raise TypeError("q, k, v must be torch.Tensor instances")
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("Input tensors must be 4-dimensional [batch, seq_len, num_heads, head_dim]")
@@ -72,9 +72,10 @@ def validate_inputs_enhanced(q, k, v, scale=None, bias=None, dropout_p=0.0):
     if q.dtype not in SUPPORTED_DTYPES:
         raise ValueError(f"Unsupported dtype {q.dtype}. Supported types: "
                          + ", ".join(str(d) for d in SUPPORTED_DTYPES))
-    if not (q.device == k.device == v.device):
+    device = q.device
+    if not (device == k.device == v.device):
         raise ValueError(f"All tensors must be on the same device. Got Q: {q.device}, K: {k.device}, V: {v.device}")
-    if q.device.type != "cuda":
+    if device.type != "cuda":
         raise ValueError("Flash Attention requires GPU tensors (there is no CPU path)")
     if bias is not None:
         if not isinstance(bias, torch.Tensor):

@@ -53,6 +53,8 @@ SUPPORTED_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 def check_block_sizes(block_size_m: Optional[int], block_size_n: Optional[int]) -> None:
     """Tile-size hints must be positive multiples of 16 no larger than 256
     (the reference rejects unusable tiles and falls back, tests/test_attention.py:602-625)."""
+    if block_size_m is None and block_size_n is None:
+        return
     for name, val in (("block_size_m", block_size_m), ("block_size_n", block_size_n)):
         if val is None:
             continue
@@ -63,19 +65,22 @@ def check_block_sizes(block_size_m: Optional[int], block_size_n: Optional[int]) 
 def _check_kernel_inputs(q, k, v, dropout_p, bias=None):
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("Input tensors must be 4-dimensional [batch, seq_len, num_heads, head_dim]")
-    if not (q.dtype == k.dtype == v.dtype) or q.dtype not in SUPPORTED_DTYPES:
+    dtype, device = q.dtype, q.device
+    if not (dtype == k.dtype == v.dtype) or dtype not in SUPPORTED_DTYPES:
         raise ValueError(f"dtype must be one of {SUPPORTED_DTYPES} and equal for q, k, v")
-    if q.device.type != "cuda" or k.device != q.device or v.device != q.device:
+    if device.type != "cuda" or k.device != device or v.device != device:
         raise ValueError("Flash Attention requires q, k, v on the same GPU device")
-    if not _lib.padded_head_dim(q.shape[-1], q.dtype, bias is not None):
+    B, _, H, D = q.shape
+    kshape = k.shape
+    if not _lib.padded_head_dim(D, dtype, bias is not None):
         raise NotImplementedError(
-            f"head_dim {q.shape[-1]} has no kernel for {q.dtype}{' with a bias' if bias is not None else ''} "
+            f"head_dim {D} has no kernel for {dtype}{' with a bias' if bias is not None else ''} "
             f"(1..{_lib.HEAD_DIMS[-1]}, and up to {_lib.WIDE_HEAD_DIM} for fp16 / bf16 without a bias; head dims "
             f"between the compiled {_lib.HEAD_DIMS + (_lib.WIDE_HEAD_DIM,)} run zero-padded to the next one)")
-    if k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[3] != q.shape[3]:
+    if kshape != v.shape or kshape[0] != B or kshape[3] != D:
         raise ValueError(f"incompatible shapes q {tuple(q.shape)}, k {tuple(k.shape)}, v {tuple(v.shape)}")
-    if k.shape[2] == 0 or q.shape[2] % k.shape[2] != 0:
-        raise ValueError(f"num_heads {q.shape[2]} must be a multiple of num_heads_kv {k.shape[2]}")
+    if kshape[2] == 0 or H % kshape[2] != 0:
+        raise ValueError(f"num_heads {H} must be a multiple of num_heads_kv {kshape[2]}")
     if not (0.0 <= dropout_p < 1.0):
         raise ValueError(f"dropout_p must be in [0.0, 1.0), got {dropout_p}")
 
