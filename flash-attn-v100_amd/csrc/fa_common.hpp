@@ -264,33 +264,59 @@ __device__ FA_INLINE inline s16x8 cat4(const s16x4& a, const s16x4& b) {
 // Philox4x32-10 (Salmon et al., SC'11) with Triton's tl.rand conventions:
 // key = (lo32 seed, hi32 seed), counter = (lo32 c, hi32 c, 0, 0); word 0 is
 // bit-cast to int32, folded x < 0 ? -x - 1 : x, and scaled by 4.6566127342e-10.
-__device__ FA_INLINE inline uint32_t philox_word0(uint64_t seed, uint64_t ctr) {
-    uint32_t c0 = (uint32_t)ctr, c1 = (uint32_t)(ctr >> 32), c2 = 0u, c3 = 0u;
-    uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+//
+// a ^ b ^ c in one instruction (v_bitop3_b32, truth table 0x96; the compiler
+// makes two xors of it: 34 of them a draw beside 18 wide multiplies, about half
+// of its cycles)
+__device__ FA_INLINE inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)c, 0x96);
+}
+// rounds FIRST .. 9 on the words c0 .. c3 (k0, k1: the key of round FIRST)
+template <int FIRST>
+__device__ FA_INLINE inline uint32_t philox_rounds(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
+                                                   uint32_t k1) {
 #pragma unroll
-    for (int r = 0; r < 10; ++r) {
+    for (int r = FIRST; r < 10; ++r) {
         // one 32 x 32 -> 64-bit product per multiplier (v_mad_u64_u32 gives
         // both halves; separate mul_hi / mul_lo cost twice the multiplies)
         const uint64_t pb = (uint64_t)0xCD9E8D57u * c2, pa = (uint64_t)0xD2511F53u * c0;
-        const uint32_t hb = (uint32_t)(pb >> 32), lb = (uint32_t)pb;
-        const uint32_t ha = (uint32_t)(pa >> 32), la = (uint32_t)pa;
-        c0 = hb ^ c1 ^ k0;
-        c2 = ha ^ c3 ^ k1;
-        c1 = lb;
-        c3 = la;
+        c0 = xor3((uint32_t)(pb >> 32), c1, k0);
+        c2 = xor3((uint32_t)(pa >> 32), c3, k1);
+        c1 = (uint32_t)pb;
+        c3 = (uint32_t)pa;
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
     return c0;
 }
+__device__ FA_INLINE inline uint32_t philox_word0(uint64_t seed, uint64_t ctr) {
+    return philox_rounds<0>((uint32_t)ctr, (uint32_t)(ctr >> 32), 0u, 0u, (uint32_t)seed, (uint32_t)(seed >> 32));
+}
+// The same for a counter whose high word is wave-uniform: words 2 and 3 are
+// zero, so word 0 after round 0 depends on the high word and the key alone, and
+// one product of round 1 and half of the xors of rounds 1 and 2 are scalar.
+__device__ FA_INLINE inline uint32_t philox_word0_hi(uint64_t seed, uint32_t hi, uint32_t lo) {
+    constexpr uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u, M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
+    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+    const uint64_t p0 = (uint64_t)M0 * lo;                   // round 0
+    const uint64_t p1a = (uint64_t)M0 * (hi ^ k0);           // round 1, uniform
+    const uint64_t p1b = (uint64_t)M1 * ((uint32_t)(p0 >> 32) ^ k1);
+    const uint32_t c0 = (uint32_t)(p1b >> 32) ^ (k0 + W0);
+    const uint32_t c2 = (uint32_t)p0 ^ ((uint32_t)(p1a >> 32) ^ (k1 + W1));
+    const uint64_t p2a = (uint64_t)M0 * c0, p2b = (uint64_t)M1 * c2;  // round 2
+    return philox_rounds<3>(xor3((uint32_t)(p2b >> 32), (uint32_t)p1b, k0 + 2 * W0), (uint32_t)p2b,
+                            (uint32_t)(p2a >> 32) ^ ((uint32_t)p1a ^ (k1 + 2 * W1)), (uint32_t)p2a, k0 + 3 * W0,
+                            k1 + 3 * W1);
+}
 
 // Keep test of the dropout mask without the float mapping: u = fp32(fold(x)) *
 // 4.6566127342e-10 (fold(x) = x < 0 ? -x - 1 : x on the int32 view) is
 // non-decreasing in fold(x), so u > p exactly when fold(x) > T, with T the
-// largest fold value whose u is <= p (keep_threshold on the host).
+// largest fold value whose u is <= p (keep_threshold on the host).  fold(x) <= T
+// is -T - 1 <= x <= T: one addition and one unsigned compare.
+__device__ FA_INLINE inline bool keep_word(uint32_t x, uint32_t thresh) { return x + thresh + 1u > 2u * thresh + 1u; }
 __device__ FA_INLINE inline bool philox_keep(uint64_t seed, uint64_t ctr, uint32_t thresh) {
-    const int32_t x = (int32_t)philox_word0(seed, ctr);
-    return (uint32_t)(x ^ (x >> 31)) > thresh;
+    return keep_word(philox_word0(seed, ctr), thresh);
 }
 
 // All ones when bit `pos` of x is set, else zero (one sign-extending

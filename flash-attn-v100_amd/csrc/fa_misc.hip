@@ -41,11 +41,16 @@ hipError_t launch_dropout_mask(uint64_t seed, uint64_t offset, int B, int H, int
 // other's multiply latency), then one ballot per (row, v) gives two words,
 // which lanes 0 and 1 store.  Under causal masking a group stops after the last
 // key any of its queries sees (the bits of keys past a query's own diagonal
-// are drawn but never read).  Rows (fewer than 2^31: B*H*Sq rows of q fit in
-// memory) use 32-bit index math.
+// are drawn but never read); the last step of a row draws only the 64-key sets
+// it needs.  Rows (fewer than 2^31: B*H*Sq rows of q fit in memory) use 32-bit
+// index math.
 // 2 rows x 4 key groups: measured against 1 x 8, 4 x 2 and 8 x 1, the best
 // balance between long rows (fewer groups per key) and short causal rows
 // (less drawn past the diagonal)
+// Bound by the vector integer rate: a draw is 17 wide multiplies (8 cycles a
+// wave each) and 17 three-way xors (4).  Measured (8 x 16 heads x 1000 x 1000,
+// causal): 144 us with two-operand xors, every product in vector registers and
+// whole 256-key steps; 95 us now
 constexpr int KB_ROWS = 2;
 constexpr int KB_SETS = 8 / KB_ROWS;
 __global__ __launch_bounds__(256) void keep_bits_kernel(uint64_t seed, uint64_t offset, uint32_t thresh,
@@ -61,25 +66,45 @@ __global__ __launch_bounds__(256) void keep_bits_kernel(uint64_t seed, uint64_t 
             const int i0 = r0 % Sq, last = min(KB_ROWS, rows - r0) - 1;
             kend = min(Sk, (i0 + last < Sq ? i0 + last : Sq - 1) + 1);
         }
-        for (int k0 = 0; k0 < kend; k0 += 64 * KB_SETS) {
-            bool keep[KB_ROWS][KB_SETS];
+        // sets keys k0 + 64 v + lane, v < SETS, of the group's rows
+        auto draw = [&](int k0, auto sets_tag) FA_INLINE {
+            constexpr int SETS = decltype(sets_tag)::value;
+            bool keep[KB_ROWS][SETS];
+#pragma unroll
+            for (int u = 0; u < KB_ROWS; ++u) {
+                // the counters of a step share their high word unless their
+                // low words wrap inside it (wave-uniform)
+                const uint64_t c0 = offset + (uint64_t)(r0 + u) * (uint64_t)Sk + (uint64_t)k0;
+                const uint32_t lo = (uint32_t)c0, hi = (uint32_t)(c0 >> 32);
+                if (lo <= 0xFFFFFFFFu - 64 * SETS) {
+#pragma unroll
+                    for (int v = 0; v < SETS; ++v)
+                        keep[u][v] = keep_word(philox_word0_hi(seed, hi, lo + 64 * v + lane), thresh);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < SETS; ++v)
+                        keep[u][v] = philox_keep(seed, c0 + (uint64_t)(64 * v + lane), thresh);
+                }
+            }
 #pragma unroll
             for (int u = 0; u < KB_ROWS; ++u)
 #pragma unroll
-                for (int v = 0; v < KB_SETS; ++v)
-                    keep[u][v] = philox_keep(
-                        seed, offset + (uint64_t)(r0 + u) * (uint64_t)Sk + (uint64_t)(k0 + 64 * v + lane), thresh);
-#pragma unroll
-            for (int u = 0; u < KB_ROWS; ++u)
-#pragma unroll
-                for (int v = 0; v < KB_SETS; ++v) {
+                for (int v = 0; v < SETS; ++v) {
                     // keys past Sk and rows past the last one draw too (never stored or read)
                     const uint64_t bal = __ballot(keep[u][v]);
                     const int w = ((k0 + 64 * v) >> 5) + lane;  // lanes 0, 1: the two 32-key words
                     if (lane < 2 && w < kb_w && r0 + u < rows)
                         kb[(int64_t)(r0 + u) * kb_w + w] = lane == 0 ? (uint32_t)bal : (uint32_t)(bal >> 32);
                 }
-        }
+        };
+        int k0 = 0;
+        for (; k0 + 64 * (KB_SETS - 1) < kend; k0 += 64 * KB_SETS) draw(k0, std::integral_constant<int, KB_SETS>{});
+        if (k0 + 128 < kend)
+            draw(k0, std::integral_constant<int, 3>{});
+        else if (k0 + 64 < kend)
+            draw(k0, std::integral_constant<int, 2>{});
+        else if (k0 < kend)
+            draw(k0, std::integral_constant<int, 1>{});
     }
 }
 
