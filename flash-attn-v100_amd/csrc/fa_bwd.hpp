@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "fa_common.hpp"
+#include "fa_f32.hpp"
 #include "fa_params.hpp"
 
 namespace fa {
@@ -2479,6 +2480,7 @@ inline bool bwd_small_runs(const BwdParams& p) {
 
 template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, typename P>
 hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
+    constexpr bool F32_PLAIN = Elem<T>::kF32 && std::is_void<TB>::value;  // the kernels of fa_f32.hpp
     if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 64 || D == 96 || D == 128)) {
         if (stage < 0 && bwd_small_runs<T, D, CAUSAL>(p0)) {
             hipError_t e = launch_bwd_t<T, D, CAUSAL, DROPOUT, TB, P>(p0, 0, s);  // delta rows
@@ -2523,6 +2525,13 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
         const int nk = (p.Sk + C::BK - 1) / C::BK;
         const int64_t nb = (int64_t)nk * p.Hkv * p.B;
         bool done = false;
+        if constexpr (F32_PLAIN) {
+            static_assert(F32Cfg<D>::BM == C::BK, "same key blocks");
+            if (nb > 0) {
+                hipLaunchKernelGGL((dkdv32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, p, nk);
+                done = true;
+            }
+        }
         if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
             if (dkdv_pp_runs(p)) {
                 using CP = DkdvPPCfg<T, D>;
@@ -2549,8 +2558,11 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
                                    s, p, nk);
             }
         } else {
-            if (!done && nb > 0)
-                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, D, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nk);
+            if constexpr (!F32_PLAIN) {
+                if (!done && nb > 0)
+                    hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, D, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0,
+                                       s, p, nk);
+            }
         }
     }
     if (stage < 0 || stage == 2) {
@@ -2558,6 +2570,13 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
         const int nq = (p.Sq + C::BM - 1) / C::BM;
         const int64_t nb = (int64_t)nq * p.H * p.B;
         bool done = false;
+        if constexpr (F32_PLAIN) {
+            static_assert(F32Cfg<D>::BM == C::BM, "same query tiles");
+            if (nb > 0) {
+                hipLaunchKernelGGL((dq32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, p, nq);
+                done = true;
+            }
+        }
         // dS stored by the dK/dV pass: dQ = scale * dS K
         if constexpr (!Elem<T>::kF32 && !std::is_void<TB>::value) {
             if (p.dq_from_ds) {
@@ -2582,15 +2601,17 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
         }
         // grids of fewer workgroups than CUs split the key loop in two inside
         // the workgroup (as the forward does) where two splits' tiles fit the LDS
-        if constexpr (2 * C::SMEM_BYTES <= 160 * 1024) {
+        if constexpr (!F32_PLAIN && 2 * C::SMEM_BYTES <= 160 * 1024) {
             if (!done && nb > 0 && nb < 256 && p.Sk > C::BN) {
                 hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 2, P>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s,
                                    p, nq);
                 done = true;
             }
         }
-        if (!done && nb > 0)
-            hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
+        if constexpr (!F32_PLAIN) {
+            if (!done && nb > 0)
+                hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
+        }
     }
     return hipGetLastError();
 }

@@ -65,6 +65,78 @@ __device__ FA_INLINE inline f32x16 mfma_f32(float a, float b, const f32x16& c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// ---------------------------------------------------------------------------
+// float32 products on the bf16 matrix instructions.  A float32 value is exactly
+// the sum of three bf16 values of its sign (its 24 mantissa bits in pieces of 8,
+// cut, not rounded, so that no piece overflows); the product of two keeps the
+// six pairs of pieces down to 2^-16 of it and drops three below 2^-22 (2^-24
+// on average), accumulated in float32.  v_mfma_f32_32x32x2_f32 takes 64 cycles
+// for 2 of the summed index, the six products 192 for 16: 2.7x the rate, of
+// which splitting the operands takes back some on the vector unit.
+struct Split3 {
+    s16x8 p[3];
+};
+// A lower piece that would be 0 (or, of an infinite value, inf - inf) is the
+// smallest normal value of the sign instead: an infinite factor then makes the
+// same infinity of every piece, as of the value itself, and a finite one adds
+// 2^-126 of itself.  NONNEG: values without a sign (P).
+template <bool NONNEG>
+__device__ FA_INLINE inline Split3 split3(const float (&x)[8]) {
+    typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
+    constexpr float tiny = 1.17549435e-38f;
+    u32x4v w[3];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float h[3][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float a = NONNEG ? x[2 * j + e] : __builtin_fabsf(x[2 * j + e]);
+            const float a0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, a) & 0xFFFF0000u);
+            const float r = fmaxf(a - a0, tiny);
+            const float a1 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, r) & 0xFFFF0000u);
+            h[0][e] = x[2 * j + e];
+            h[1][e] = r;
+            h[2][e] = fmaxf(r - a1, tiny);
+        }
+#pragma unroll
+        for (int t = 0; t < 3; ++t)  // the upper halves of two floats
+            w[t][j] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, h[t][1]), __builtin_bit_cast(unsigned, h[t][0]),
+                                            0x07060302u);
+        if constexpr (!NONNEG) {  // the signs
+            w[1][j] |= w[0][j] & 0x80008000u;
+            w[2][j] |= w[0][j] & 0x80008000u;
+        }
+    }
+    Split3 s;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) s.p[t] = __builtin_bit_cast(s16x8, w[t]);
+    return s;
+}
+// c + a b, 16 of the summed index (operand layout of v_mfma_f32_32x32x16_bf16).
+// SWAP: the pieces in the order mfma_split(b, a) takes them: S = Q K^T of the
+// dK/dV kernel then has the bits of the S^T = K Q^T whose LSE it subtracts
+// (large scores: the rounding of S cancels; dV at q, k of standard deviation 4,
+// 2 x 777 x 8 heads of 64: 2-norm error 5.7e-6 with another order in the
+// forward, 2.0e-6 with the same in all three).
+template <bool SWAP = false>
+__device__ FA_INLINE inline f32x16 mfma_split(const Split3& a, const Split3& b, f32x16 c) {
+    constexpr int X = SWAP ? 0 : 1;
+    c = Elem<bf16>::mfma(a.p[2 * X], b.p[2 - 2 * X], c);
+    c = Elem<bf16>::mfma(a.p[2 - 2 * X], b.p[2 * X], c);
+    c = Elem<bf16>::mfma(a.p[1], b.p[1], c);
+    c = Elem<bf16>::mfma(a.p[X], b.p[1 - X], c);
+    c = Elem<bf16>::mfma(a.p[1 - X], b.p[X], c);
+    return Elem<bf16>::mfma(a.p[0], b.p[0], c);
+}
+// eight consecutive floats (two 16-byte loads) split
+__device__ FA_INLINE inline Split3 split3_row(const f32x4& u, const f32x4& v) {
+    const float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
+    return split3<false>(x);
+}
+__device__ FA_INLINE inline Split3 split3_row(const uint4& u, const uint4& v) {
+    return split3_row(__builtin_bit_cast(f32x4, u), __builtin_bit_cast(f32x4, v));
+}
+
 // 8 x 16-bit elements <-> 8 floats
 template <typename T>
 __device__ FA_INLINE inline s16x8 pack8(const float* x) {

@@ -19,7 +19,9 @@
 //   * causal: KV tiles past the last query are never loaded; tiles past a
 //     wave's last query are skipped by that wave; only diagonal and tail tiles
 //     run the masking variant of the tile step.
-//   * fp32 inputs use v_mfma_f32_32x32x2_f32 with fp32 P.
+//   * fp32 inputs run the same products on their values cut into three bf16
+//     pieces where they are read (mfma_split), P too (grids that fill the
+//     chip, without a bias: fwd32_kernel of fa_f32.hpp).
 //   * optional additive bias (BIAS): each lane reads 4 consecutive keys of its
 //     query's bias row per load, issued a tile ahead; the scores become
 //     t = S * scale + bias (one FMA) before the mask, and the softmax runs on
@@ -29,6 +31,7 @@
 #include <type_traits>
 
 #include "fa_common.hpp"
+#include "fa_f32.hpp"
 #include "fa_params.hpp"
 
 namespace fa {
@@ -119,13 +122,15 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         const T* qrow = (const T*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh;
 #pragma unroll
         for (int i = 0; i < QR; ++i) {
-            // bf16/f16: d = 16i + 8hi .. +7 ; f32: d = hi*D/2 + 4i .. +3
-            const int d0 = C::F32 ? hi * (D / 2) + 4 * i : 16 * i + 8 * hi;
+            // bf16/f16: d = 16i + 8hi .. +7 ; f32: half of that each, in the order of
+            // fwd32_kernel and the fp32 backward (S with the same bits)
+            const int d0 = C::F32 ? 16 * (i >> 1) + 8 * hi + 4 * (i & 1) : 16 * i + 8 * hi;
             qreg[i] = qi < p.Sq && d0 < ncols<D>(p) ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
     }
     // no wait here: the Q loads stay in flight while the first tile copies
     // are issued (the barrier before the first product waits for both)
+    Split3 qsp[C::F32 ? D / 16 : 1];  // fp32: Q in pieces, cut once the copies are issued
 
     f32x16 o[D / 32];
 #pragma unroll
@@ -247,11 +252,10 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
             const T* krow = Ks + (32 * blk + l32) * KW;
             if constexpr (C::F32) {
 #pragma unroll
-                for (int i = 0; i < QR; ++i) {
-                    const f32x4 a = *reinterpret_cast<const f32x4*>(krow + hi * (D / 2) + 4 * i);
-                    const f32x4 bq = __builtin_bit_cast(f32x4, qreg[i]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) s[blk] = mfma_f32(a[e], bq[e], s[blk]);
+                for (int kk = 0; kk < D / 16; ++kk) {
+                    const T* kp = krow + 16 * kk + 8 * hi;
+                    const Split3 a = split3_row(*reinterpret_cast<const f32x4*>(kp), *reinterpret_cast<const f32x4*>(kp + 4));
+                    s[blk] = mfma_split(a, qsp[kk], s[blk]);
                 }
             } else {
 #pragma unroll
@@ -336,13 +340,20 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     auto pv = [&](const T* Vs, const f32x16 (&s)[NB], const s16x8 (&pk)[NPK]) {
         if constexpr (C::F32) {
 #pragma unroll
-            for (int blk = 0; blk < NB; ++blk)
+            for (int ks = 0; ks < BN / 16; ++ks) {
+                float ps[8];
 #pragma unroll
-                for (int t = 0; t < 16; ++t) {
-                    const T* vrow = Vs + (32 * blk + 8 * (t >> 2) + 4 * hi + (t & 3)) * VW + l32;
+                for (int e = 0; e < 8; ++e) ps[e] = s[ks >> 1][8 * (ks & 1) + e];
+                const Split3 bp = split3<true>(ps);
 #pragma unroll
-                    for (int i = 0; i < D / 32; ++i) o[i] = mfma_f32(vrow[32 * i], s[blk][t], o[i]);
+                for (int i = 0; i < D / 32; ++i) {
+                    float vs[8];  // the keys of the lane's P values, column 32 i + l32
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        vs[e] = Vs[(16 * ks + 8 * (e >> 2) + 4 * hi + (e & 3)) * VW + 32 * i + l32];
+                    o[i] = mfma_split(split3<false>(vs), bp, o[i]);
                 }
+            }
         } else {
 #pragma unroll
             for (int ks = 0; ks < BN / 16; ++ks)
@@ -393,6 +404,10 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         dma_k(0, 0);
         dma_k(1, 1);
         load_v(0, 0);
+    }
+    if constexpr (C::F32) {
+#pragma unroll
+        for (int kk = 0; kk < D / 16; ++kk) qsp[kk] = split3_row(qreg[2 * kk], qreg[2 * kk + 1]);
     }
     sync_tiles();
     if (n_w > 0) {
@@ -916,6 +931,17 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
                 if (host_group_uneven(32, q.n_qtiles, (int)nblocks)) return launch_fwd_pp_fit<T>(q, nblocks, s);
             }
             hipLaunchKernelGGL((fwd_pp_kernel<T, D, CAUSAL, false, P>), dim3((unsigned)nblocks), dim3(CP::NT), 0, s, q);
+            return hipGetLastError();
+        }
+    }
+    // grids that fill the CUs; smaller ones split the key loop (below), where
+    // the two forms take the same time and the split sums are more accurate
+    if constexpr (Elem<T>::kF32 && std::is_void<TB>::value) {
+        P q = p;
+        q.n_qtiles = (p.Sq + F32Cfg<D>::BM - 1) / F32Cfg<D>::BM;
+        const int64_t nb = (int64_t)q.n_qtiles * p.H * p.B;
+        if (nb >= 256) {
+            hipLaunchKernelGGL((fwd32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, q);
             return hipGetLastError();
         }
     }
