@@ -19,9 +19,9 @@
 //   * causal: KV tiles past the last query are never loaded; tiles past a
 //     wave's last query are skipped by that wave; only diagonal and tail tiles
 //     run the masking variant of the tile step.
-//   * fp32 inputs run the same products on their values cut into three bf16
-//     pieces where they are read (mfma_split), P too (grids that fill the
-//     chip, without a bias: fwd32_kernel of fa_f32.hpp).
+//   * fp32 inputs with a bias use v_mfma_f32_32x32x2_f32 with fp32 P; without
+//     one their values are cut into three bf16 pieces where they are read
+//     (mfma_split), P too (grids that fill the chip: fwd32_kernel, fa_f32.hpp).
 //   * optional additive bias (BIAS): each lane reads 4 consecutive keys of its
 //     query's bias row per load, issued a tile ahead; the scores become
 //     t = S * scale + bias (one FMA) before the mask, and the softmax runs on
@@ -75,6 +75,9 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     using BT = typename std::conditional<BIAS, TB, T>::type;
     constexpr int BN = C::BN, NB = C::NB, KW = C::KW, VW = C::VW;
     constexpr bool BIAS_LDS = QG > 1;
+    // fp32 products on bf16 pieces, as the fp32 backward without a bias takes
+    // them (with a bias both stay on the fp32 instruction: S with the same bits)
+    constexpr bool SPLIT = C::F32 && !BIAS;
     static_assert(QG == 1 || (QG == 2 && BIAS && !Elem<BT>::kF32 && !C::F32 && DROPOUT == 0 && KS == 1 && BN == 64),
                   "query groups: the staged 16-bit bias path");
     constexpr int BREG = 32 * 64;  // elements of a wave's bias region (32 rows of 64 keys)
@@ -122,15 +125,15 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         const T* qrow = (const T*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh;
 #pragma unroll
         for (int i = 0; i < QR; ++i) {
-            // bf16/f16: d = 16i + 8hi .. +7 ; f32: half of that each, in the order of
-            // fwd32_kernel and the fp32 backward (S with the same bits)
-            const int d0 = C::F32 ? 16 * (i >> 1) + 8 * hi + 4 * (i & 1) : 16 * i + 8 * hi;
+            // bf16/f16: d = 16i + 8hi .. +7 ; f32: half of that each (SPLIT), or
+            // d = hi*D/2 + 4i .. +3: the orders of the backward's S, for the same bits
+            const int d0 = SPLIT ? 16 * (i >> 1) + 8 * hi + 4 * (i & 1) : C::F32 ? hi * (D / 2) + 4 * i : 16 * i + 8 * hi;
             qreg[i] = qi < p.Sq && d0 < ncols<D>(p) ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0u, 0u, 0u, 0u);
         }
     }
     // no wait here: the Q loads stay in flight while the first tile copies
     // are issued (the barrier before the first product waits for both)
-    Split3 qsp[C::F32 ? D / 16 : 1];  // fp32: Q in pieces, cut once the copies are issued
+    Split3 qsp[SPLIT ? D / 16 : 1];  // fp32: Q in pieces, cut once the copies are issued
 
     f32x16 o[D / 32];
 #pragma unroll
@@ -250,7 +253,15 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         for (int blk = 0; blk < NB; ++blk) {
             s[blk] = f32x16{};
             const T* krow = Ks + (32 * blk + l32) * KW;
-            if constexpr (C::F32) {
+            if constexpr (C::F32 && !SPLIT) {
+#pragma unroll
+                for (int i = 0; i < QR; ++i) {
+                    const f32x4 a = *reinterpret_cast<const f32x4*>(krow + hi * (D / 2) + 4 * i);
+                    const f32x4 bq = __builtin_bit_cast(f32x4, qreg[i]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[blk] = mfma_f32(a[e], bq[e], s[blk]);
+                }
+            } else if constexpr (SPLIT) {
 #pragma unroll
                 for (int kk = 0; kk < D / 16; ++kk) {
                     const T* kp = krow + 16 * kk + 8 * hi;
@@ -338,7 +349,16 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     };
     // ---- O^T += V^T P^T ----
     auto pv = [&](const T* Vs, const f32x16 (&s)[NB], const s16x8 (&pk)[NPK]) {
-        if constexpr (C::F32) {
+        if constexpr (C::F32 && !SPLIT) {
+#pragma unroll
+            for (int blk = 0; blk < NB; ++blk)
+#pragma unroll
+                for (int t = 0; t < 16; ++t) {
+                    const T* vrow = Vs + (32 * blk + 8 * (t >> 2) + 4 * hi + (t & 3)) * VW + l32;
+#pragma unroll
+                    for (int i = 0; i < D / 32; ++i) o[i] = mfma_f32(vrow[32 * i], s[blk][t], o[i]);
+                }
+        } else if constexpr (SPLIT) {
 #pragma unroll
             for (int ks = 0; ks < BN / 16; ++ks) {
                 float ps[8];
@@ -405,7 +425,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         dma_k(1, 1);
         load_v(0, 0);
     }
-    if constexpr (C::F32) {
+    if constexpr (SPLIT) {
 #pragma unroll
         for (int kk = 0; kk < D / 16; ++kk) qsp[kk] = split3_row(qreg[2 * kk], qreg[2 * kk + 1]);
     }
