@@ -2434,14 +2434,23 @@ __global__ __launch_bounds__(256, 2) void dq_ds_kernel(const BwdParams p, const 
 // 64): on grids of fewer workgroups than CUs, whose serial tile chain its two
 // waves per SIMD halve, and with a bias at every grid size (two waves per SIMD
 // where dkdv_kernel fits one), unless dkdv_kernel's per-element zero fill of
-// the causal dBias is needed (rows not 16-byte aligned).
+// the causal dBias is needed (rows not 16-byte aligned).  Causal grids of up to
+// two workgroups per CU run for the chains of their first keys too; backward in
+// us with dkdv_kernel and dkdv8_kernel (bf16; workgroups, queries): D = 128
+// (384, 2048) 160 / 133, (384, 4096) 333 / 277, (320, 1024) 89.9 / 75.2; D = 64 (384, 700) 40.3 / 38.3, (384, 512) 34.8 / 36.5, (384,
+// 2048) 88.4 / 81.2, (512, 2048) 95.8 / 93.3, (512, 1024) 58.0 / 59.1; chains of
+// one length lose ((384, 1024) full, 71 / 79).  At D = 128 shorter chains keep
+// dkdv_kernel, whose results equal the ping-pong kernel's bit for bit.
 template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB>
 inline bool dkdv8_runs(const BwdParams& p) {
     if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && D >= 64 && D <= 128) {
         constexpr bool BIAS = !std::is_void<TB>::value;
         const int64_t nb = (int64_t)((p.Sk + DkdvCfg<T, D>::BK - 1) / DkdvCfg<T, D>::BK) * p.Hkv * p.B;
         const bool fill1 = BIAS && CAUSAL && p.dbias != nullptr && p.dbias_zero_fill == 1;
-        return nb > 0 && (nb < 256 || BIAS) && !fill1;
+        const int seen = p.Sq < p.Sk ? p.Sq : p.Sk;
+        const bool chain = CAUSAL && (nb <= 256 || (nb <= 400 && seen >= (D > 64 ? 1536 : 700)) ||
+                                      (D == 64 && nb <= 512 && seen >= 2048));
+        return nb > 0 && (nb < 256 || BIAS || chain) && !fill1;
     }
     return false;
 }
@@ -2461,19 +2470,37 @@ inline bool dq_pp_runs(const BwdParams& p) {
     return nb >= 256;
 }
 
+// Whether dq_kernel splits the key loop inside its workgroups: grids of fewer
+// workgroups than CUs, and causal grids (without bias or dropout, where
+// measured) bound by their longest rows' chains.  Causal backward in us without
+// and with it (bf16; workgroups, keys): D = 64 (384, 4096) 184 / 164, (512, 4096)
+// 171 / 167, (384, 1024) 51.1 / 53.6; D = 128 (384, 2048) 133 / 127, (384, 1024)
+// 80.6 / 86.0; D = 32 (256, 512) 23.8 / 23.5, (256, 4096) 119 / 110, (512, 2048)
+// 70.4 / 70.1, (512, 1024) 41.5 / 42.6.  256: as bwd_small_kernel's.
+template <bool CAUSAL>
+inline bool dq_splits_keys(const BwdParams& p, int64_t nb, bool plain) {
+    if (nb < 256) return true;
+    const int seen = p.Sq < p.Sk ? p.Sq : p.Sk;
+    return CAUSAL && plain && (nb == 256 || (nb <= 512 && seen >= 2048));
+}
+
 // Whether the whole backward runs as the delta pre-pass plus bwd_small_kernel
 // (16-bit inputs, D = 64 to 128, no bias or dropout): where dK/dV would run
-// dkdv8_kernel on fewer workgroups than CUs and dQ the key-split dq_kernel,
-// and either both kinds of workgroups fit the CUs at once or the mask makes
-// their tile chains uneven (non-causal chains of one length on more workgroups
-// than CUs gain nothing from sharing them and would pay the pre-pass).
+// dkdv8_kernel on at most as many workgroups as CUs and dQ the key-split
+// dq_kernel, and either both kinds of workgroups fit the CUs at once or the mask
+// makes their tile chains uneven (non-causal chains of one length on more
+// workgroups than CUs gain nothing from sharing them and would pay the
+// pre-pass).  Causal, 256 workgroups of each kind, us of the two passes and of
+// this launch: D = 64 4096 queries 158 / 107, 1024 47.5 / 38.2, 512 30.3 / 28.2;
+// D = 128 280 / 154, 85 / 55, 53 / 43; 384 of each: 206 / 184, where the passes
+// with dkdv8_kernel and key-split dQ take 164.
 template <typename T, int D, bool CAUSAL>
 inline bool bwd_small_runs(const BwdParams& p) {
     if constexpr (!Elem<T>::kF32 && (D == 64 || D == 96 || D == 128) && 2 * DqCfg<T, D>::SMEM_BYTES <= 160 * 1024) {
         const int64_t nq = (int64_t)((p.Sq + DqCfg<T, D>::BM - 1) / DqCfg<T, D>::BM) * p.H * p.B;
         const int64_t nkv = (int64_t)((p.Sk + Dkdv8Cfg<T, D>::BK - 1) / Dkdv8Cfg<T, D>::BK) * p.Hkv * p.B;
-        return dkdv8_runs<T, D, CAUSAL, 0, void>(p) && nq > 0 && nq < 256 && p.Sk > DqCfg<T, D>::BN &&
-               (CAUSAL || nq + nkv <= 256);
+        return dkdv8_runs<T, D, CAUSAL, 0, void>(p) && nq > 0 && p.Sk > DqCfg<T, D>::BN &&
+               (CAUSAL ? nq <= 256 && nkv <= 256 : nq + nkv <= 256);
     }
     return false;
 }
@@ -2599,10 +2626,10 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
                 done = true;
             }
         }
-        // grids of fewer workgroups than CUs split the key loop in two inside
-        // the workgroup (as the forward does) where two splits' tiles fit the LDS
+        // split the key loop in two inside the workgroup (as the forward does)
+        // where two splits' tiles fit the LDS
         if constexpr (!F32_PLAIN && 2 * C::SMEM_BYTES <= 160 * 1024) {
-            if (!done && nb > 0 && nb < 256 && p.Sk > C::BN) {
+            if (!done && nb > 0 && dq_splits_keys<CAUSAL>(p, nb, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
                 hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 2, P>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s,
                                    p, nq);
                 done = true;

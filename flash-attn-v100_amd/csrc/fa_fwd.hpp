@@ -937,6 +937,24 @@ inline bool fwd_pp_wanted(const FwdParams& p, bool causal) {
     return n >= 256 && (!causal || (p.Sq >= 3072 && n >= 512));
 }
 
+// Whether fwd_kernel splits the key loop inside its workgroups (KS): grids of
+// fewer workgroups than CUs, and causal grids (without bias or dropout, where
+// measured) of up to two workgroups per CU whose longest rows are long: they
+// run for the length of those chains while most workgroups have ended.  Causal,
+// us without and with the split (bf16; workgroups, keys): D = 64 (256, 512)
+// 12.7 / 12.1, (256, 2048) 29.3 / 24.7, (384, 1024) 19.1 / 20.4, (384, 2048)
+// 30.8 / 26.9, (384, 4096) 76 / 57, (512, 2048) 32.8 / 32.1; D = 128 (256, 1024)
+// 24.9 / 24.6, (384, 2048) 46.1 / 44.3, (512, 2048) 50.7 / 53.3, (512, 4096)
+// 91.6 / 88.0; full rows of one length lose 5-30% ((384, 1024) 28.8 / 32.8).
+template <int D, bool CAUSAL>
+inline bool fwd_splits_keys(int64_t nblocks, int Sq, int Sk, bool plain) {
+    if (nblocks < 256) return true;
+    if (!CAUSAL || !plain) return false;
+    const int keys = Sq < Sk ? Sq : Sk;  // that the last query sees
+    if (nblocks == 256) return keys >= (D > 64 ? 1024 : 512);
+    return nblocks <= 512 && keys >= (D > 64 && nblocks > 400 ? 4096 : 2048);
+}
+
 template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, typename P>
 hipError_t launch_fwd_t(const P& p, hipStream_t s) {
     if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
@@ -984,14 +1002,13 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
     q.n_qtiles = (p.Sq + C::BM - 1) / C::BM;
     const int64_t nblocks = (int64_t)q.n_qtiles * p.H * p.B;
     if (nblocks <= 0) return hipSuccess;
-    // grids that leave CUs idle split the key loop inside the workgroup: into
+    // split the key loop inside the workgroup (fwd_splits_keys): into
     // 4 where four splits fit 128 registers a lane without spilling (16-bit,
     // D = 32, no dropout, no bias), else into 2
     constexpr int KS_SMALL = (!Elem<T>::kF32 && D == 32 && DROPOUT == 0 && std::is_void<TB>::value) ? 4 : 2;
-    const int n_cu = 256;
     // (D = 256: one workgroup's tiles take most of the LDS, no split)
     if constexpr (D <= 128) {
-        if (nblocks < n_cu && p.Sk > C::BN) {
+        if (fwd_splits_keys<D, CAUSAL>(nblocks, p.Sq, p.Sk, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
             hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, KS_SMALL, 1, P>), dim3((unsigned)nblocks),
                                dim3(C::NT * KS_SMALL), 0, s, q);
             return hipGetLastError();
