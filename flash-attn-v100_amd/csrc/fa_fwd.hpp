@@ -68,20 +68,24 @@ struct FwdCfg {
 // region: 16-byte copies along the rows, where per-lane loads (one query row
 // per lane) touch 32 rows per instruction.  The LDS of one such workgroup
 // holds the K/V tiles and the 8 bias regions.
-template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, int QG = 1, typename P = FwdParams>
+// STAGED: the bias through LDS, with query groups or with a key split (D <= 64:
+// two splits' tiles and 8 regions fit the LDS).
+template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, int KS, int QG = 1, typename P = FwdParams,
+          bool STAGED = (QG > 1)>
 __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 : 1) void fwd_kernel(const P p) {
     using C = FwdCfg<T, D>;
     constexpr bool BIAS = !std::is_void<TB>::value;
     using BT = typename std::conditional<BIAS, TB, T>::type;
     constexpr int BN = C::BN, NB = C::NB, KW = C::KW, VW = C::VW;
-    constexpr bool BIAS_LDS = QG > 1;
+    constexpr bool BIAS_LDS = STAGED;
     // fp32 products on bf16 pieces, as the fp32 backward without a bias takes
     // them (with a bias both stay on the fp32 instruction: S with the same bits)
     constexpr bool SPLIT = C::F32 && !BIAS;
-    static_assert(QG == 1 || (QG == 2 && BIAS && !Elem<BT>::kF32 && !C::F32 && DROPOUT == 0 && KS == 1 && BN == 64),
-                  "query groups: the staged 16-bit bias path");
+    static_assert(QG == 1 || (QG == 2 && STAGED && KS == 1), "query groups stage the bias");
+    static_assert(!STAGED || (BIAS && !Elem<BT>::kF32 && !C::F32 && DROPOUT == 0 && BN == 64),
+                  "the staged 16-bit bias path");
     constexpr int BREG = 32 * 64;  // elements of a wave's bias region (32 rows of 64 keys)
-    __shared__ __attribute__((aligned(16))) T smem[C::SMEM_ELEMS * KS + (BIAS_LDS ? 4 * QG * BREG : 0)];
+    __shared__ __attribute__((aligned(16))) T smem[C::SMEM_ELEMS * KS + (BIAS_LDS ? 4 * KS * QG * BREG : 0)];
 
     const int tid = threadIdx.x;
     // wave index as a scalar: loop bounds derived from it stay wave-uniform;
@@ -984,11 +988,29 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
         }
     }
     using C = FwdCfg<T, D>;
-    // a 16-bit bias without dropout: 256-query workgroups that stage the bias
-    // through LDS, where the grid still fills the CUs and bias rows are whole
-    // 16-byte chunks
+    // a 16-bit bias without dropout, bias rows of whole 16-byte chunks: staged
+    // through LDS, by 256-query workgroups where the grid still fills the CUs
     if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && !std::is_void<TB>::value) {
         if constexpr (!Elem<TB>::kF32) {
+            // small grids split the key loop with the bias staged too: grids of at
+            // most one workgroup per CU, and causal ones of up to two with long
+            // chains, whose 256-query workgroups (or unstaged splits) run for the
+            // length of their longest key loop.  us before and after (bf16, D = 64;
+            // 128-query workgroups, keys): (256, 2048) 55.7 / 34.8, full 57.5 / 34.6,
+            // (192, 2048) 48.1 / 33.9, (256, 512) 17.5 / 13.8, (64, 256) 11.1 / 10.1;
+            // causal (512, 2048) 58.1 / 46.3, (512, 1024) 32.6 / 29.8, (512, 512)
+            // 20.6 / 21.5; full (512, 1024) 33.0 / 39.1
+            if constexpr (D <= 64) {
+                P q = p;
+                q.n_qtiles = (p.Sq + C::BM - 1) / C::BM;
+                const int64_t nb1 = (int64_t)q.n_qtiles * p.H * p.B;
+                const bool split = nb1 <= 256 || (CAUSAL && nb1 <= 512 && (p.Sq < p.Sk ? p.Sq : p.Sk) >= 1024);
+                if (split && nb1 > 0 && p.Sk % 8 == 0 && p.Sk > C::BN) {
+                    hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, 0, TB, 2, 1, P, true>), dim3((unsigned)nb1), dim3(C::NT * 2),
+                                       0, s, q);
+                    return hipGetLastError();
+                }
+            }
             P q = p;
             q.n_qtiles = (p.Sq + 2 * C::BM - 1) / (2 * C::BM);
             const int64_t nb2 = (int64_t)q.n_qtiles * p.H * p.B;
