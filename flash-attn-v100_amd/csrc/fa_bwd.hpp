@@ -2643,7 +2643,7 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
     return hipGetLastError();
 }
 
-// head dims between the compiled ones (p.head_cols; fa_cols.hpp)
+// head dims between the compiled ones (p.head_cols), instantiated in fa_bwd_cols_*.hip
 template <typename T>
 hipError_t launch_bwd_cols(const BwdParams& p, int D, bool causal, int stage, hipStream_t s);
 template <typename T>

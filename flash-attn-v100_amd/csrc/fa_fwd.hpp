@@ -1043,7 +1043,7 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
 // The few-row forward (fa_fwd_decode.hpp, instantiated in fa_fwd_decode.hip)
 template <typename T>
 hipError_t launch_fwd_decode(const FwdParams& p, int D, bool causal, hipStream_t s);
-// head dims between the compiled ones (p.head_cols; fa_cols.hpp)
+// head dims between the compiled ones (p.head_cols), instantiated in fa_fwd_cols_*.hip
 template <typename T>
 hipError_t launch_fwd_cols(const FwdParams& p, int D, bool causal, hipStream_t s);
 
