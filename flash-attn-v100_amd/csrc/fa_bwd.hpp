@@ -677,7 +677,7 @@ __global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const P p, const int n_
     const uint64_t chead = opaque64((uint64_t)(grp == 0 ? p.q_sh : p.do_sh) * sizeof(T));  // bytes per head
     const uint64_t wbase = opaque64((uint64_t)(uintptr_t)(p.lse2 + (int64_t)b * p.H * p.ws_stride));
     const uint32_t wrow_bytes = opaque32((uint32_t)p.ws_stride * 4u);
-    const uint32_t full_bytes = opaque32((uint32_t)(((BQ - 1) * (int)css + D) * (int)sizeof(T)));
+    const uint32_t full_bytes = opaque32((uint32_t)(((BQ - 1) * (int)css + ncols<D>(p)) * (int)sizeof(T)));
     const uint32_t woff = 4u * (uint32_t)(grp * p.sq_pad + lane);
     const int q_rows = p.Sq;
     // per-lane source offsets of the wave's row-copy items 8 n + 4 hf + w4
@@ -702,7 +702,8 @@ __global__ __launch_bounds__(512, 1) void dkdv_pp_kernel(const P p, const int n_
     };
     const int qb0_first = (qt_end - 1) * BQ;
     const uint32_t bytes_first = opaque32(
-        q_rows - qb0_first >= BQ ? full_bytes : (uint32_t)(((q_rows - qb0_first - 1) * (int)css + D) * (int)sizeof(T)));
+        q_rows - qb0_first >= BQ ? full_bytes
+                                 : (uint32_t)(((q_rows - qb0_first - 1) * (int)css + ncols<D>(p)) * (int)sizeof(T)));
     const uint32_t wbytes_first = opaque32(wrow_bytes - 4u * (uint32_t)qb0_first);
     const uint64_t dsrc = opaque64((uint64_t)BQ * crow);
     const uint32_t lds_first = __builtin_amdgcn_readfirstlane(lds_addr(smem + grp * C::QALLOC));
@@ -1957,7 +1958,7 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const P p) {
     const uint64_t cbase = opaque64((uint64_t)(uintptr_t)(grp == 0 ? (const T*)p.k + b * p.k_sb + hk * p.k_sh
                                                                    : (const T*)p.v + b * p.v_sb + hk * p.v_sh));
     const uint64_t crow = opaque64((uint64_t)css * sizeof(T));
-    const uint32_t full_bytes = (uint32_t)(((BN - 1) * (int)css + D) * (int)sizeof(T));
+    const uint32_t full_bytes = (uint32_t)(((BN - 1) * (int)css + ncols<D>(p)) * (int)sizeof(T));
     const int n_copy = (C::NI - w4 + 3) / 4;  // this wave's instructions per tile (wave-uniform)
     int coff[C::PER];
 #pragma unroll
@@ -1972,8 +1973,9 @@ __global__ __launch_bounds__(512, 1) void dq_pp_kernel(const P p) {
     // tile j < n_tiles at source src, LDS address l0: the keys [j BN, min(Sk, j BN + BN)),
     // rows past Sk land as zeros (only the last tile can be partial)
     const uint32_t last_bytes = opaque32(
-        p.Sk - (n_tiles - 1) * BN >= BN ? full_bytes
-                                        : (uint32_t)(((p.Sk - (n_tiles - 1) * BN - 1) * (int)css + D) * (int)sizeof(T)));
+        p.Sk - (n_tiles - 1) * BN >= BN
+            ? full_bytes
+            : (uint32_t)(((p.Sk - (n_tiles - 1) * BN - 1) * (int)css + ncols<D>(p)) * (int)sizeof(T)));
     auto issue_at = [&](int j, uint64_t src, uint32_t l0) FA_INLINE {
         u32x4 rs;
         rs[0] = (uint32_t)src;

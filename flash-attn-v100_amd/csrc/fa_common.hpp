@@ -14,6 +14,8 @@
 
 #include <type_traits>
 
+#include "fa_params.hpp"
+
 // Device helpers and kernel-local lambdas are always inlined: an out-of-line
 // call would keep tile descriptors and MFMA accumulators in scratch memory
 // (and turn wave-uniform buffer descriptors into per-lane ones).
@@ -489,18 +491,19 @@ __device__ FA_INLINE inline int2 slice_bh(int s, int NH, int B, bool head_major)
 
 // ---------------------------------------------------------------------------
 // Raw buffer view of the rows [0, min(nvalid, R)) of a tile of R rows in a
-// row-strided [rows][D] slice: loads at byte offsets past the last valid row
-// return zeros (hardware range check), which zero-fills tail tiles without any
-// per-lane branch or select.  The descriptor is rebuilt per tile (base
-// advanced to the tile, record count bounded by the tile's rows), so the range
-// check never depends on the scalar offset and only tile-local offsets need 32
-// bits: the host bounds the byte span of kTileRows rows below 2^31, whatever
-// the length of the whole slice.  The byte count is computed without a branch
+// row-strided [rows][cols] slice (cols: the columns that exist, D where all
+// do): loads at byte offsets past the last valid row return zeros (hardware
+// range check), which zero-fills tail tiles without any per-lane branch or
+// select.  The descriptor is rebuilt per tile (base advanced to the tile,
+// record count bounded by the tile's rows: tile_bytes), so the range check
+// never depends on the scalar offset and only tile-local offsets need 32 bits:
+// the host bounds the byte span of kTileRows rows below 2^31, whatever the
+// length of the whole slice.  The byte count is computed without a branch
 // (nvalid <= 0 gives 0) so that a tile load does not end a basic block.
 template <typename T, int D, int R>
-__device__ FA_INLINE inline __amdgpu_buffer_rsrc_t row_buffer(const T* base, int64_t row_stride, int nvalid) {
-    const int nv = min(max(nvalid, 0), R);
-    const int bytes = ((nv - 1) * (int)row_stride + D) * (int)sizeof(T) * min(nv, 1);
+__device__ FA_INLINE inline __amdgpu_buffer_rsrc_t row_buffer(const T* base, int64_t row_stride, int nvalid,
+                                                              int cols = D) {
+    const int bytes = tile_bytes(nvalid, R, (int)row_stride, cols, (int)sizeof(T));
     // dword 3: DATA_FORMAT = 32 (untyped dword access), no swizzle, no stride
     return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)bytes, 0x00020000);
 }
@@ -565,10 +568,8 @@ __device__ FA_INLINE inline u32x4 buffer_words(const void* base, int bytes) {
 // Four-dword buffer descriptor of the rows [0, min(nvalid, R)) of a tile, as
 // row_buffer builds it (raw untyped dword access, no stride, no swizzle).
 template <typename T, int D, int R>
-__device__ FA_INLINE inline u32x4 row_buffer_words(const T* base, int64_t row_stride, int nvalid) {
-    const int nv = min(max(nvalid, 0), R);
-    const int bytes = ((nv - 1) * (int)row_stride + D) * (int)sizeof(T) * min(nv, 1);
-    return buffer_words(base, bytes);
+__device__ FA_INLINE inline u32x4 row_buffer_words(const T* base, int64_t row_stride, int nvalid, int cols = D) {
+    return buffer_words(base, tile_bytes(nvalid, R, (int)row_stride, cols, (int)sizeof(T)));
 }
 
 // LDS byte address of a __shared__ object (an address-space cast, then the
@@ -600,13 +601,15 @@ struct DmaTile {
     static constexpr int PER = (NI + NW - 1) / NW;
     int off[PER];
     int wave;
+    int cols;  // the columns that exist
 
     // wave_id must be wave-uniform (readfirstlane): it selects the LDS
     // destination, which the hardware takes from a scalar register (M0).
-    // cols: the columns that exist (at most D, whole 16-byte chunks); the
+    // n_cols: the columns that exist (at most D, whole 16-byte chunks); the
     // others land as zeros
-    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int cols = D) {
+    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int n_cols = D) {
         wave = wave_id;
+        cols = n_cols;
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int c = 64 * (wave + NW * t) + lane;
@@ -616,7 +619,7 @@ struct DmaTile {
         }
     }
     __device__ FA_INLINE inline void load(const T* base, int64_t row_stride, int nvalid, T* lds, int lane) const {
-        const __amdgpu_buffer_rsrc_t rs = row_buffer<T, D, R>(base, row_stride, nvalid);
+        const __amdgpu_buffer_rsrc_t rs = row_buffer<T, D, R>(base, row_stride, nvalid, cols);
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int g = wave + NW * t;
@@ -630,7 +633,7 @@ struct DmaTile {
     // the caller waits for it (vmcnt) before the barrier that publishes it
     __device__ FA_INLINE inline void load_untracked(const T* base, int64_t row_stride, int nvalid, const T* lds,
                                                     int lane) const {
-        load_words(row_buffer_words<T, D, R>(base, row_stride, nvalid), lds);
+        load_words(row_buffer_words<T, D, R>(base, row_stride, nvalid, cols), lds);
     }
     // the same untracked copy through a caller-built descriptor (whose range
     // ends where the readable data ends; chunks past it land as zeros)
@@ -717,9 +720,11 @@ struct DmaRowGroups {
     int off;   // byte offset of this lane's chunk within its row group
     int rowl;  // this lane's row within the group (KR for idle lanes)
     int wave;
+    int cols;  // the columns that exist, as in DmaTile
 
-    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int cols = D) {
+    __device__ FA_INLINE inline void init(int64_t row_stride, int lane, int wave_id, int n_cols = D) {
         wave = wave_id;
+        cols = n_cols;
         rowl = lane < KR * CW ? lane / CW : KR;
         // padding chunks read nothing: an offset past the range stays past it
         // (below 2^32) after the group's row step is added (tiles span < 2^31
@@ -728,7 +733,7 @@ struct DmaRowGroups {
         off = col < cols / EPC ? ((lane / CW) * (int)row_stride + col * EPC) * (int)sizeof(T) : kOffNowhere;
     }
     __device__ FA_INLINE inline void load(const T* base, int64_t row_stride, int nvalid, T* lds) const {
-        const __amdgpu_buffer_rsrc_t rs = row_buffer<T, D, R>(base, row_stride, nvalid);
+        const __amdgpu_buffer_rsrc_t rs = row_buffer<T, D, R>(base, row_stride, nvalid, cols);
 #pragma unroll
         for (int t = 0; t < PER; ++t) {
             const int g = wave + NWAVES * t;
@@ -743,7 +748,7 @@ struct DmaRowGroups {
     // Idle lanes (past the group's rows) are switched off by the branch, which
     // masks exec around the assembly.
     __device__ FA_INLINE inline void load_untracked(const T* base, int64_t row_stride, int nvalid, const T* lds) const {
-        const u32x4 rs = row_buffer_words<T, D, R>(base, row_stride, nvalid);
+        const u32x4 rs = row_buffer_words<T, D, R>(base, row_stride, nvalid, cols);
         const uint32_t l0 = lds_addr(lds);
 #pragma unroll
         for (int t = 0; t < PER; ++t) {

@@ -7,6 +7,17 @@
 
 namespace fa {
 
+// Bytes of the rows [0, min(nvalid, rows)) of a tile, from the first row's first
+// element to the last row's last one of `cols` that exist: the range of the
+// tile's buffer descriptor.  It must not reach row nvalid, which starts `stride`
+// >= cols elements after the row before it: that row belongs to another head,
+// to the unfilled part of a cache or to no tensor, and lands as zeros.  No
+// branch; 0 for nvalid <= 0.
+__host__ __device__ constexpr int tile_bytes(int nvalid, int rows, int stride, int cols, int elem) {
+    const int n0 = nvalid > 0 ? nvalid : 0, nv = n0 < rows ? n0 : rows;
+    return ((nv - 1) * stride + cols) * elem * (nv < 1 ? nv : 1);
+}
+
 // Strides are in elements; the d stride is 1 (checked by the host shim).
 struct FwdParams {
     const void* q;

@@ -295,6 +295,21 @@ static void bwd_paths() {
     t = a; t.dropout_p = 3.f; CHECK(fa_bwd_static(&t, nullptr) == FA_ERR_DROPOUT);
 }
 
+// The range of a tile descriptor never reaches the row behind the last valid
+// one, whatever columns exist and however close the rows follow, and never
+// loses a valid element: every head dim that runs at a wider compiled one.
+static void tile_ranges() {
+    for (int cols = 40; cols <= 248; cols += 8)
+        for (int stride = cols; stride <= cols + 264; stride += 8)
+            for (int rows : {32, 64})
+                for (int nv = -3; nv <= rows + 3; ++nv) {
+                    const int n = nv < 0 ? 0 : nv < rows ? nv : rows;
+                    const int bytes = fa::tile_bytes(nv, rows, stride, cols, 2);
+                    CHECK(bytes == (n == 0 ? 0 : ((n - 1) * stride + cols) * 2));
+                    CHECK(bytes <= n * stride * 2);  // where row n begins
+                }
+}
+
 static void misc() {
     for (int c = -20; c <= 2; ++c) CHECK(fa_strerror(c) != nullptr && std::strlen(fa_strerror(c)) > 0);
     CHECK(fa_abi_version() == FA_ABI_VERSION);
@@ -312,6 +327,7 @@ int main() {
     fwd_valid();
     fwd_rejects();
     bwd_paths();
+    tile_ranges();
     misc();
     for (void* p : g_bufs) std::free(p);
     std::printf("%d checks, %d failed\n", g_cases, g_fails);
