@@ -177,6 +177,11 @@ __global__ __launch_bounds__(256, ((std::is_void<TB>::value || D <= 64) && !(Ele
     const int k0 = kt * C::BK;
     const int kw0 = k0 + 32 * w;
     const int kj = kw0 + l32;  // this lane's key
+    // float32 without a bias: only the rows that dkdv32_kernel has left
+    if constexpr (C::F32 && !BIAS) {
+        const float* first = (const float*)p.dk + b * p.dk_sb + (int64_t)k0 * p.dk_ss + hk * p.dk_sh;
+        if (*reinterpret_cast<const unsigned*>(first) != kRedo) return;
+    }
 
     // ---- K, V rows of this lane's key in registers (MFMA B operands) ----
     constexpr int KR = C::F32 ? D / 8 : D / 16;
@@ -1406,6 +1411,11 @@ __device__ FA_INLINE inline void dq_body(const P& p, const int n_qtiles, const i
     const int q0 = qt * C::BM;
     const int qw0 = q0 + 32 * w;
     const int qi = qw0 + l32;
+    // float32 without a bias: only the rows that dq32_kernel has left
+    if constexpr (C::F32 && !BIAS) {
+        const float* first = (const float*)p.dq + b * p.dq_sb + (int64_t)q0 * p.dq_ss + h * p.dq_sh;
+        if (*reinterpret_cast<const unsigned*>(first) != kRedo) return;
+    }
 
     constexpr int QR = C::F32 ? D / 8 : D / 16;
     const bool own_delta = !C::F32 && p.dq_delta;
@@ -2558,7 +2568,6 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
             static_assert(F32Cfg<D>::BM == C::BK, "same key blocks");
             if (nb > 0) {
                 hipLaunchKernelGGL((dkdv32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, p, nk);
-                done = true;
             }
         }
         if constexpr (!Elem<T>::kF32 && DROPOUT == 0 && std::is_void<TB>::value && (D == 128 || D == 96)) {
@@ -2587,11 +2596,10 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
                                    s, p, nk);
             }
         } else {
-            if constexpr (!F32_PLAIN) {
-                if (!done && nb > 0)
-                    hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, D, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0,
-                                       s, p, nk);
-            }
+            // (float32 without a bias: the rows that dkdv32_kernel left)
+            if (!done && nb > 0)
+                hipLaunchKernelGGL((dkdv_kernel<T, D, CAUSAL, DROPOUT, TB, D, 0, P>), dim3((unsigned)nb), dim3(C::NT), 0, s,
+                                   p, nk);
         }
     }
     if (stage < 0 || stage == 2) {
@@ -2603,7 +2611,6 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
             static_assert(F32Cfg<D>::BM == C::BM, "same query tiles");
             if (nb > 0) {
                 hipLaunchKernelGGL((dq32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, p, nq);
-                done = true;
             }
         }
         // dS stored by the dK/dV pass: dQ = scale * dS K
@@ -2637,10 +2644,9 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
                 done = true;
             }
         }
-        if constexpr (!F32_PLAIN) {
-            if (!done && nb > 0)
-                hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
-        }
+        // (float32 without a bias: the rows that dq32_kernel left)
+        if (!done && nb > 0)
+            hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, p, nq);
     }
     return hipGetLastError();
 }

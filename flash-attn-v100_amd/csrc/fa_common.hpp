@@ -69,44 +69,35 @@ __device__ FA_INLINE inline f32x16 mfma_f32(float a, float b, const f32x16& c) {
 
 // ---------------------------------------------------------------------------
 // float32 products on the bf16 matrix instructions.  A float32 value is exactly
-// the sum of three bf16 values of its sign (its 24 mantissa bits in pieces of 8,
-// cut, not rounded, so that no piece overflows); the product of two keeps the
-// six pairs of pieces down to 2^-16 of it and drops three below 2^-22 (2^-24
-// on average), accumulated in float32.  v_mfma_f32_32x32x2_f32 takes 64 cycles
-// for 2 of the summed index, the six products 192 for 16: 2.7x the rate, of
-// which splitting the operands takes back some on the vector unit.
+// the sum of three bf16 values: the value rounded to bf16, the rest rounded to
+// bf16, and what is left then (24 mantissa bits in signed pieces of 8).  The
+// product of two values keeps the six pairs of pieces down to 2^-16 of it; the
+// three dropped are at most 2^-24 of it (2^-27 in the root mean square, of
+// either sign).
+// v_mfma_f32_32x32x2_f32 takes 64 cycles for 2 of the summed index, the six
+// products 192 for 16: 2.7x the rate, of which splitting the operands takes
+// back some on the vector unit.
+// Zeros stay zeros, NaN stay NaN.  Pieces end at 2^-133 (the smallest bf16; the
+// instructions keep denormal values, in and out, as the float32 one does), and
+// an infinity has none: workgroups that meet a value which they do not carry
+// (PieceRange) leave their rows to a kernel on v_mfma_f32_32x32x2_f32.
 struct Split3 {
     s16x8 p[3];
 };
-// A lower piece that would be 0 (or, of an infinite value, inf - inf) is the
-// smallest normal value of the sign instead: an infinite factor then makes the
-// same infinity of every piece, as of the value itself, and a finite one adds
-// 2^-126 of itself.  NONNEG: values without a sign (P).
-template <bool NONNEG>
 __device__ FA_INLINE inline Split3 split3(const float (&x)[8]) {
     typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
-    constexpr float tiny = 1.17549435e-38f;
+    typedef float f32x2v __attribute__((ext_vector_type(2)));
+    typedef bf16 bf16x2v __attribute__((ext_vector_type(2)));
     u32x4v w[3];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        float h[3][2];
+        f32x2v r = {x[2 * j], x[2 * j + 1]};
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const float a = NONNEG ? x[2 * j + e] : __builtin_fabsf(x[2 * j + e]);
-            const float a0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, a) & 0xFFFF0000u);
-            const float r = fmaxf(a - a0, tiny);
-            const float a1 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, r) & 0xFFFF0000u);
-            h[0][e] = x[2 * j + e];
-            h[1][e] = r;
-            h[2][e] = fmaxf(r - a1, tiny);
-        }
-#pragma unroll
-        for (int t = 0; t < 3; ++t)  // the upper halves of two floats
-            w[t][j] = __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, h[t][1]), __builtin_bit_cast(unsigned, h[t][0]),
-                                            0x07060302u);
-        if constexpr (!NONNEG) {  // the signs
-            w[1][j] |= w[0][j] & 0x80008000u;
-            w[2][j] |= w[0][j] & 0x80008000u;
+        for (int t = 0; t < 3; ++t) {
+            const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2v));
+            w[t][j] = h;
+            r[0] -= __builtin_bit_cast(float, h << 16);
+            r[1] -= __builtin_bit_cast(float, h & 0xFFFF0000u);
         }
     }
     Split3 s;
@@ -114,7 +105,61 @@ __device__ FA_INLINE inline Split3 split3(const float (&x)[8]) {
     for (int t = 0; t < 3; ++t) s.p[t] = __builtin_bit_cast(s16x8, w[t]);
     return s;
 }
-// c + a b, 16 of the summed index (operand layout of v_mfma_f32_32x32x16_bf16).
+// Collects whether a value is neither zero nor NaN nor of a magnitude in
+// [2^-100, 2^30).  Within that range pieces are exact and nothing overflows, up
+// to products of three values; values of dO V^T and dS below 2^-110 lose what
+// is below 2^-133 of them.  Two vector instructions a value.
+struct PieceRange {
+    unsigned lo = ~0u;  // smallest 2 |x| - 1 as an integer: zeros wrap to the largest
+    unsigned hi = 0u;   // largest |x|, as an integer
+    // x passes through the assembly, so that it is looked at before it is cut:
+    // otherwise the compiler does that last and keeps every x until then (40
+    // registers more, up to 1.4 KiB of scratch)
+    __device__ FA_INLINE inline void add(float (&x)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            unsigned a, b;
+            asm("v_max3_f32 %0, |%2|, |%3|, %0\n\t"
+                "v_lshl_add_u32 %4, %2, 1, -1\n\t"
+                "v_lshl_add_u32 %5, %3, 1, -1\n\t"
+                "v_min3_u32 %1, %4, %5, %1"
+                : "+v"(hi), "+v"(lo), "+v"(x[e]), "+v"(x[e + 1]), "=&v"(a), "=&v"(b));
+        }
+    }
+    // a row's delta: dS overflows with it (O was infinite, or huge)
+    __device__ FA_INLINE inline void add_delta(float d) {
+        hi = max(hi, __builtin_bit_cast(unsigned, __builtin_fabsf(d) * 0x1p-60f));
+    }
+    __device__ FA_INLINE inline bool odd() const {
+        return lo < 2u * ((127u - 100u) << 23) - 1u || hi >= (127u + 30u) << 23;
+    }
+};
+// In place of the first value that a workgroup would write (a NaN of its own):
+// its rows are for the kernel on the float32 instruction, launched after it,
+// whose other workgroups end at once.  A result that happens to be this NaN is
+// computed again, no more.
+constexpr unsigned kRedo = 0x7FC5A3E1u;
+// whether a thread of the workgroup has met such a value: put before a barrier,
+// read after it (one slot per wave, NW a multiple of 4)
+__device__ FA_INLINE inline void put_odd(unsigned* flags, const PieceRange& range, int wave, int lane) {
+    const bool odd = __ballot(range.odd()) != 0ull;
+    if (lane == 0) flags[wave] = odd ? 1u : 0u;
+}
+template <int NW>
+__device__ FA_INLINE inline bool any_odd(const unsigned* flags) {
+    unsigned f = 0u;
+#pragma unroll
+    for (int i = 0; i < NW; i += 4) {
+        const uint4 x = *reinterpret_cast<const uint4*>(flags + i);
+        f |= x.x | x.y | x.z | x.w;
+    }
+    return __builtin_amdgcn_readfirstlane(f) != 0u;
+}
+// c + a b, 16 of the summed index (operand layout of v_mfma_f32_32x32x16_bf16),
+// the smallest products first.  The instruction cuts a c below its products at
+// their last place instead of rounding, so the score of one product can be an
+// ulp off; the largest first rounds right there, but five more times (error
+// over whole calls 6-30% larger).
 // SWAP: the pieces in the order mfma_split(b, a) takes them: S = Q K^T of the
 // dK/dV kernel then has the bits of the S^T = K Q^T whose LSE it subtracts
 // (large scores: the rounding of S cancels; dV at q, k of standard deviation 4,
@@ -130,15 +175,6 @@ __device__ FA_INLINE inline f32x16 mfma_split(const Split3& a, const Split3& b, 
     c = Elem<bf16>::mfma(a.p[1 - X], b.p[X], c);
     return Elem<bf16>::mfma(a.p[0], b.p[0], c);
 }
-// eight consecutive floats (two 16-byte loads) split
-__device__ FA_INLINE inline Split3 split3_row(const f32x4& u, const f32x4& v) {
-    const float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
-    return split3<false>(x);
-}
-__device__ FA_INLINE inline Split3 split3_row(const uint4& u, const uint4& v) {
-    return split3_row(__builtin_bit_cast(f32x4, u), __builtin_bit_cast(f32x4, v));
-}
-
 // 8 x 16-bit elements <-> 8 floats
 template <typename T>
 __device__ FA_INLINE inline s16x8 pack8(const float* x) {

@@ -1,6 +1,9 @@
 // Forward, dQ and dK/dV for float32 inputs without a bias on the bf16 matrix
 // instructions: every operand is cut into three bf16 pieces (split3) and a
-// product is six matrix products of pieces (mfma_split).
+// product is six matrix products of pieces (mfma_split).  A workgroup that
+// meets a value out of their range writes a mark (kRedo) in place of its first
+// result and nothing else; fwd_kernel, dq_kernel and dkdv_kernel, launched
+// after these kernels over the same blocks of rows, compute the marked ones.
 //
 // fwd_kernel, dq_kernel and dkdv_kernel run float32 on
 // v_mfma_f32_32x32x2_f32, whose rate bounds them (fp32 matrix peak is 1/16 of
@@ -12,13 +15,16 @@
 // read like 16-bit tiles (rows, or columns with ds_read_b64_tr_b16).  One LDS
 // buffer and two barriers a tile: the workgroups of a CU cover each other's.
 // Bound by the matrix products and the splitting of P / dS per tile.
-// Error against 64 bits (largest 2-norm over O, dQ, dK, dV at 8 x 1000 x 16
-// heads of 64): 2.7e-7, 4.1e-7, 4.1e-7,
-// 3.6e-7 (on v_mfma_f32_32x32x2_f32: 3.2e-7, 4.9e-7, 5.0e-7, 4.3e-7).
-// Measured (forward / dQ and dK/dV, us; before: on v_mfma_f32_32x32x2_f32):
-// 8 x 1000 x 16 heads of 64, full: 294 / 924 -> 223 / 661; causal with dropout,
-// step of 32 / 64 / 128 columns: bwd 343 / 597 / 1209 -> 253 / 421 / 964; 4 x
-// 1024 x 16 heads of 128, full: 290 / 989 -> 214 / 772.
+// Error against 64 bits (2-norm of O, dQ, dK, dV at 8 x 1000 x 16 heads of 64):
+// full 5.4e-7, 4.7e-7, 4.6e-7, 4.4e-7 (on v_mfma_f32_32x32x2_f32 6.4e-7, 7.6e-7,
+// 7.5e-7, 7.3e-7), causal 2.6e-7, 3.6e-7, 3.6e-7, 3.0e-7 (3.3e-7, 4.8e-7, 4.9e-7,
+// 4.2e-7).
+// Measured (forward / dQ and dK/dV, us; before: on v_mfma_f32_32x32x2_f32; the
+// kernels for marked rows, of which there are none here, are 1 to 2 of each):
+// 8 x 1000 x 16 heads of 64, full: 288 / 916 -> 203 / 635; causal with dropout,
+// heads of 32, 64, 128: 225 / 324, 307 / 595, 457 / 1213 -> 156 / 229, 199 /
+// 405, 361 / 993; 4 x 1024 x 16 heads of 128, full: 262 / 982 -> 199 / 686.
+// Small grids too: 1 x 512 x 8 heads of 64 39 / 129 -> 35 / 98.
 #pragma once
 
 #include "fa_common.hpp"
@@ -68,7 +74,7 @@ struct F32Stage {
         }
     }
     // the pieces into the tiles la, lb
-    __device__ FA_INLINE inline void store(bf16* la, bf16* lb, int tid) const {
+    __device__ FA_INLINE inline void store(bf16* la, bf16* lb, int tid, PieceRange& range) const {
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
             const int c = tid + C::NT * u;
@@ -76,8 +82,9 @@ struct F32Stage {
             const int cc = c - (second ? CH : 0);
             bf16* dst = (second ? lb : la) + (cc / CPR) * C::RW + (cc % CPR) * 8;
             const f32x4 p = __builtin_bit_cast(f32x4, x[u][0]), q = __builtin_bit_cast(f32x4, x[u][1]);
-            const float v[8] = {p[0], p[1], p[2], p[3], q[0], q[1], q[2], q[3]};
-            const Split3 s = split3<false>(v);
+            float v[8] = {p[0], p[1], p[2], p[3], q[0], q[1], q[2], q[3]};
+            range.add(v);
+            const Split3 s = split3(v);
 #pragma unroll
             for (int t = 0; t < 3; ++t) *reinterpret_cast<s16x8*>(dst + t * D) = s.p[t];
         }
@@ -104,7 +111,8 @@ __device__ FA_INLINE inline Split3 f32_col_frag(const bf16* tile, int ks, int i,
 }
 // a row of D floats in registers: pieces of columns 16 kk + 8 hi .. + 7 (zeros if !ok)
 template <int D>
-__device__ FA_INLINE inline void f32_row_regs(const float* row, bool ok, int hi, Split3 (&s)[D / 16]) {
+__device__ FA_INLINE inline void f32_row_regs(const float* row, bool ok, int hi, Split3 (&s)[D / 16],
+                                                    PieceRange& range) {
 #pragma unroll
     for (int kk = 0; kk < D / 16; ++kk) {
         float v[8];
@@ -116,16 +124,16 @@ __device__ FA_INLINE inline void f32_row_regs(const float* row, bool ok, int hi,
             v[e + 2] = x.z;
             v[e + 3] = x.w;
         }
-        s[kk] = split3<false>(v);
+        range.add(v);
+        s[kk] = split3(v);
     }
 }
-// pieces of accumulator values 8 ks .. 8 ks + 7 (probabilities: NONNEG; dS)
-template <bool NONNEG>
+// pieces of accumulator values 8 ks .. 8 ks + 7 (P, dS)
 __device__ FA_INLINE inline Split3 f32_acc_frag(const f32x16& s, int ks) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = s[8 * ks + e];
-    return split3<NONNEG>(v);
+    return split3(v);
 }
 // acc (transposed: lane = row l32, value 4 g + e of block i = column 32 i + 8 g
 // + 4 hi + e) times mul to `rows` rows at `out`, 32 columns at a time through
@@ -160,6 +168,7 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const FwdParams p) {
     using C = F32Cfg<D>;
     constexpr int BN = C::BN;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
+    __shared__ __attribute__((aligned(16))) unsigned flags[C::NW];
     bf16* Ks = (bf16*)smem;
     bf16* Vs = Ks + C::TILE;
 
@@ -179,13 +188,14 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const FwdParams p) {
     if (CAUSAL) n_w = min(n_tiles, (qw0 + 31) / BN + 1);
 
     F32Stage<D> st;
+    PieceRange range;
     auto load = [&](int j) FA_INLINE {
         const int k0 = j * BN;
         st.load(kbase + (int64_t)k0 * p.k_ss, p.k_ss, vbase + (int64_t)k0 * p.v_ss, p.v_ss, p.Sk - k0, tid);
     };
     if (n_tiles > 0) load(0);
     Split3 qs[D / 16];
-    f32_row_regs<D>((const float*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh, qi < p.Sq, hi, qs);
+    f32_row_regs<D>((const float*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh, qi < p.Sq, hi, qs, range);
 
     f32x16 o[D / 32];
 #pragma unroll
@@ -199,7 +209,7 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const FwdParams p) {
     for (int j = 0; j < n_tiles; ++j) {
         const int k0 = j * BN;
         lds_barrier();  // every wave is done with tile j - 1
-        st.store(Ks, Vs, tid);
+        st.store(Ks, Vs, tid, range);
         uint32_t kword = 0;
         if (DROPOUT == 2 && qi < p.Sq) kword = kbrow[j];
         if (j + 1 < n_tiles) load(j + 1);
@@ -246,10 +256,16 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const FwdParams p) {
         l_run += psum;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const Split3 bp = f32_acc_frag<true>(s, ks);
+            const Split3 bp = f32_acc_frag(s, ks);
 #pragma unroll
             for (int i = 0; i < D / 32; ++i) o[i] = mfma_split(f32_col_frag<D>(Vs, ks, i, lane, hi), bp, o[i]);
         }
+    }
+    put_odd(flags, range, w, lane);
+    lds_barrier();  // every wave is done with the tiles
+    if (any_odd<C::NW>(flags)) {
+        if (tid == 0) reinterpret_cast<unsigned*>(p.lse)[(int64_t)(b * p.H + h) * p.Sq + q0] = kRedo;
+        return;
     }
     const float l_tot = pair_sum(l_run);
     const float inv = l_tot > 0.f ? (DROPOUT ? p.rp : 1.f) / l_tot : 0.f;
@@ -258,7 +274,6 @@ __global__ __launch_bounds__(256, 2) void fwd32_kernel(const FwdParams p) {
         p.lse[si] = l_tot > 0.f ? (m_run + __log2f(l_tot)) * kLn2 : -INFINITY;
         if (p.mx) p.mx[si] = m_raw * p.scale;
     }
-    lds_barrier();  // every wave is done with the tiles
     f32_store_rows<D>((float*)p.o + b * p.o_sb + h * p.o_sh + (int64_t)qw0 * p.o_ss, p.o_ss, p.Sq - qw0, o, inv,
                       (float*)smem + w * 32 * C::OW, lane, l32, hi);
 }
@@ -271,6 +286,7 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dq32_kernel(const BwdP
     using C = F32Cfg<D>;
     constexpr int BN = C::BN;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
+    __shared__ __attribute__((aligned(16))) unsigned flags[C::NW];
     bf16* Ks = (bf16*)smem;
     bf16* Vs = Ks + C::TILE;
 
@@ -290,16 +306,18 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dq32_kernel(const BwdP
     if (CAUSAL) n_w = min(n_tiles, (qw0 + 31) / BN + 1);
 
     F32Stage<D> st;
+    PieceRange range;
     auto load = [&](int j) FA_INLINE {
         const int k0 = j * BN;
         st.load(kbase + (int64_t)k0 * p.k_ss, p.k_ss, vbase + (int64_t)k0 * p.v_ss, p.v_ss, p.Sk - k0, tid);
     };
     if (n_tiles > 0) load(0);
     Split3 qs[D / 16], dos[D / 16];
-    f32_row_regs<D>((const float*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh, qi < p.Sq, hi, qs);
-    f32_row_regs<D>((const float*)p.dout + b * p.do_sb + (int64_t)qi * p.do_ss + h * p.do_sh, qi < p.Sq, hi, dos);
+    f32_row_regs<D>((const float*)p.q + b * p.q_sb + (int64_t)qi * p.q_ss + h * p.q_sh, qi < p.Sq, hi, qs, range);
+    f32_row_regs<D>((const float*)p.dout + b * p.do_sb + (int64_t)qi * p.do_ss + h * p.do_sh, qi < p.Sq, hi, dos, range);
     const int64_t wi = ((int64_t)b * p.H + h) * p.ws_stride + qi;  // qi < sq_pad
     const float lse2 = p.lse2[wi], del = p.delta[wi], c = p.scale_log2;
+    range.add_delta(del);
     uint64_t row_ctr = 0;
     if (DROPOUT == 1) row_ctr = p.offset + ((uint64_t)(b * p.H + h) * (uint64_t)p.Sq + (uint64_t)qi) * (uint64_t)p.Sk;
     const uint32_t* kbrow = p.kb + (DROPOUT == 2 && qi < p.Sq ? ((int64_t)(b * p.H + h) * p.Sq + qi) * p.kb_w : 0);
@@ -310,7 +328,7 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dq32_kernel(const BwdP
     for (int j = 0; j < n_tiles; ++j) {
         const int k0 = j * BN;
         lds_barrier();
-        st.store(Ks, Vs, tid);
+        st.store(Ks, Vs, tid, range);
         uint32_t kword = 0;
         if (DROPOUT == 2 && qi < p.Sq) kword = kbrow[j];
         if (j + 1 < n_tiles) load(j + 1);
@@ -340,15 +358,27 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dq32_kernel(const BwdP
                 s[r] = pv * (dp[r] - del);
             }
         }
+        // a tile's products summed by themselves, then added: fewer roundings at
+        // the size of dQ (error of dQ at 2 x 777 x 8 heads of 64, full: 5.9e-7
+        // summed in place, 4.2e-7; on the float32 instruction 5.8e-7)
+        const Split3 bs[2] = {f32_acc_frag(s, 0), f32_acc_frag(s, 1)};
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const Split3 bs = f32_acc_frag<false>(s, ks);
+        for (int i = 0; i < D / 32; ++i) {
+            f32x16 t = f32x16{};
 #pragma unroll
-            for (int i = 0; i < D / 32; ++i) dq[i] = mfma_split(f32_col_frag<D>(Ks, ks, i, lane, hi), bs, dq[i]);
+            for (int ks = 0; ks < 2; ++ks) t = mfma_split(f32_col_frag<D>(Ks, ks, i, lane, hi), bs[ks], t);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) dq[i][r] += t[r];
         }
     }
+    put_odd(flags, range, w, lane);
     lds_barrier();
-    f32_store_rows<D>((float*)p.dq + b * p.dq_sb + h * p.dq_sh + (int64_t)qw0 * p.dq_ss, p.dq_ss, p.Sq - qw0, dq, p.scale,
+    float* const out = (float*)p.dq + b * p.dq_sb + h * p.dq_sh;
+    if (any_odd<C::NW>(flags)) {
+        if (tid == 0) *reinterpret_cast<unsigned*>(out + (int64_t)q0 * p.dq_ss) = kRedo;
+        return;
+    }
+    f32_store_rows<D>(out + (int64_t)qw0 * p.dq_ss, p.dq_ss, p.Sq - qw0, dq, p.scale,
                       (float*)smem + w * 32 * C::OW, lane, l32, hi);
 }
 
@@ -362,6 +392,7 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dkdv32_kernel(const Bw
     constexpr int BQ = C::BN;
     __shared__ __attribute__((aligned(16))) char smem[C::SMEM_BYTES];
     __shared__ __attribute__((aligned(16))) float ws[2][BQ];  // LSE * log2 e and delta of the tile
+    __shared__ __attribute__((aligned(16))) unsigned flags[C::NW];
     bf16* Qs = (bf16*)smem;
     bf16* Ds = Qs + C::TILE;
 
@@ -376,6 +407,7 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dkdv32_kernel(const Bw
     const int total = nq * p.group;
 
     F32Stage<D> st;
+    PieceRange range;
     float wx = 0.f;
     auto load = [&](int it) FA_INLINE {
         const int hh = hk * p.group + it / nq, qb0 = (qt_end - 1 - it % nq) * BQ;
@@ -387,8 +419,8 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dkdv32_kernel(const Bw
     };
     if (total > 0) load(0);
     Split3 ksp[D / 16], vsp[D / 16];
-    f32_row_regs<D>((const float*)p.k + b * p.k_sb + (int64_t)kj * p.k_ss + hk * p.k_sh, kj < p.Sk, hi, ksp);
-    f32_row_regs<D>((const float*)p.v + b * p.v_sb + (int64_t)kj * p.v_ss + hk * p.v_sh, kj < p.Sk, hi, vsp);
+    f32_row_regs<D>((const float*)p.k + b * p.k_sb + (int64_t)kj * p.k_ss + hk * p.k_sh, kj < p.Sk, hi, ksp, range);
+    f32_row_regs<D>((const float*)p.v + b * p.v_sb + (int64_t)kj * p.v_ss + hk * p.v_sh, kj < p.Sk, hi, vsp, range);
     f32x16 dk[D / 32], dv[D / 32];
 #pragma unroll
     for (int i = 0; i < D / 32; ++i) {
@@ -399,8 +431,9 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dkdv32_kernel(const Bw
     for (int it = 0; it < total; ++it) {
         const int hh = hk * p.group + it / nq, qb0 = (qt_end - 1 - it % nq) * BQ;
         lds_barrier();
-        st.store(Qs, Ds, tid);
+        st.store(Qs, Ds, tid, range);
         if (tid < 2 * BQ) ws[tid >> 5][tid & (BQ - 1)] = wx;
+        if (tid >= BQ && tid < 2 * BQ) range.add_delta(wx);
         // the forward's keep word of query qb0 + l32 for the wave's 32 keys
         uint32_t kword = 0;
         if (DROPOUT == 2 && qb0 + l32 < p.Sq && kw0 < p.Sk)
@@ -440,19 +473,32 @@ __global__ __launch_bounds__(256, F32Cfg<D>::BLOCKS) void dkdv32_kernel(const Bw
                 dp[r] = DROPOUT ? pv * __builtin_fmaf(dpv, p.rp, -d4[e]) : pv * (dpv - d4[e]);
             }
         }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const Split3 bp = f32_acc_frag<true>(s, ks), bs = f32_acc_frag<false>(dp, ks);
+        // (each tile's products summed by themselves, as dq32_kernel does: 1-5% of
+        // the time; error of dK at 8 x 1000 x 16 heads of 64, causal: 4.2e-7 in
+        // place, 3.6e-7)
+        auto add = [&](f32x16 (&acc)[D / 32], const bf16* tile, const f32x16& x) FA_INLINE {
+            const Split3 bx[2] = {f32_acc_frag(x, 0), f32_acc_frag(x, 1)};
 #pragma unroll
             for (int i = 0; i < D / 32; ++i) {
-                dv[i] = mfma_split(f32_col_frag<D>(Ds, ks, i, lane, hi), bp, dv[i]);
-                dk[i] = mfma_split(f32_col_frag<D>(Qs, ks, i, lane, hi), bs, dk[i]);
+                f32x16 t = f32x16{};
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) t = mfma_split(f32_col_frag<D>(tile, ks, i, lane, hi), bx[ks], t);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[i][r] += t[r];
             }
-        }
+        };
+        add(dv, Ds, s);
+        add(dk, Qs, dp);
     }
+    put_odd(flags, range, w, lane);
     lds_barrier();
+    float* const out = (float*)p.dk + b * p.dk_sb + hk * p.dk_sh;
+    if (any_odd<C::NW>(flags)) {
+        if (tid == 0) *reinterpret_cast<unsigned*>(out + (int64_t)k0 * p.dk_ss) = kRedo;
+        return;
+    }
     float* stage = (float*)smem + w * 32 * C::OW;
-    f32_store_rows<D>((float*)p.dk + b * p.dk_sb + hk * p.dk_sh + (int64_t)kw0 * p.dk_ss, p.dk_ss, p.Sk - kw0, dk, p.scale,
+    f32_store_rows<D>(out + (int64_t)kw0 * p.dk_ss, p.dk_ss, p.Sk - kw0, dk, p.scale,
                       stage, lane, l32, hi);
     f32_store_rows<D>((float*)p.dv + b * p.dv_sb + hk * p.dv_sh + (int64_t)kw0 * p.dv_ss, p.dv_ss, p.Sk - kw0, dv,
                       DROPOUT ? p.rp : 1.f, stage, lane, l32, hi);

@@ -19,9 +19,11 @@
 //   * causal: KV tiles past the last query are never loaded; tiles past a
 //     wave's last query are skipped by that wave; only diagonal and tail tiles
 //     run the masking variant of the tile step.
-//   * fp32 inputs with a bias use v_mfma_f32_32x32x2_f32 with fp32 P; without
-//     one their values are cut into three bf16 pieces where they are read
-//     (mfma_split), P too (grids that fill the chip: fwd32_kernel, fa_f32.hpp).
+//   * fp32 inputs use v_mfma_f32_32x32x2_f32 with fp32 P, except that without a
+//     bias the key-split form (small grids) cuts the values into three bf16
+//     pieces where they are read (mfma_split), P too; grids that fill the chip
+//     run fwd32_kernel (fa_f32.hpp).  The unsplit form then computes the rows
+//     that these two leave to it (kRedo).
 //   * optional additive bias (BIAS): each lane reads 4 consecutive keys of its
 //     query's bias row per load, issued a tile ahead; the scores become
 //     t = S * scale + bias (one FMA) before the mask, and the softmax runs on
@@ -79,8 +81,10 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     constexpr int BN = C::BN, NB = C::NB, KW = C::KW, VW = C::VW;
     constexpr bool BIAS_LDS = STAGED;
     // fp32 products on bf16 pieces, as the fp32 backward without a bias takes
-    // them (with a bias both stay on the fp32 instruction: S with the same bits)
-    constexpr bool SPLIT = C::F32 && !BIAS;
+    // them (with a bias both stay on the fp32 instruction: S with the same
+    // bits), and the rows that such a kernel has left
+    constexpr bool SPLIT = C::F32 && !BIAS && KS > 1, REDO = C::F32 && !BIAS && KS == 1;
+    static_assert(!SPLIT || KS == 2, "flag slots of 8 waves");
     static_assert(QG == 1 || (QG == 2 && STAGED && KS == 1), "query groups stage the bias");
     static_assert(!STAGED || (BIAS && !Elem<BT>::kF32 && !C::F32 && DROPOUT == 0 && BN == 64),
                   "the staged 16-bit bias path");
@@ -107,6 +111,10 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     const int q0 = qt * C::BM * QG;  // the workgroup's first query
     const int qw0 = q0 + C::BM * qg + 32 * w;
     const int qi = qw0 + l32;
+
+    if constexpr (REDO) {
+        if (reinterpret_cast<const unsigned*>(p.lse)[(int64_t)(b * p.H + h) * p.Sq + q0] != kRedo) return;
+    }
 
     const T* __restrict__ kbase = (const T*)p.k + b * p.k_sb + hk * p.k_sh;
     const T* __restrict__ vbase = (const T*)p.v + b * p.v_sb + hk * p.v_sh;
@@ -138,6 +146,7 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     // no wait here: the Q loads stay in flight while the first tile copies
     // are issued (the barrier before the first product waits for both)
     Split3 qsp[SPLIT ? D / 16 : 1];  // fp32: Q in pieces, cut once the copies are issued
+    PieceRange range;
 
     f32x16 o[D / 32];
 #pragma unroll
@@ -269,8 +278,10 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
 #pragma unroll
                 for (int kk = 0; kk < D / 16; ++kk) {
                     const T* kp = krow + 16 * kk + 8 * hi;
-                    const Split3 a = split3_row(*reinterpret_cast<const f32x4*>(kp), *reinterpret_cast<const f32x4*>(kp + 4));
-                    s[blk] = mfma_split(a, qsp[kk], s[blk]);
+                    const f32x4 u = *reinterpret_cast<const f32x4*>(kp), v = *reinterpret_cast<const f32x4*>(kp + 4);
+                    float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
+                    range.add(x);
+                    s[blk] = mfma_split(split3(x), qsp[kk], s[blk]);
                 }
             } else {
 #pragma unroll
@@ -368,14 +379,15 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
                 float ps[8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) ps[e] = s[ks >> 1][8 * (ks & 1) + e];
-                const Split3 bp = split3<true>(ps);
+                const Split3 bp = split3(ps);
 #pragma unroll
                 for (int i = 0; i < D / 32; ++i) {
                     float vs[8];  // the keys of the lane's P values, column 32 i + l32
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
                         vs[e] = Vs[(16 * ks + 8 * (e >> 2) + 4 * hi + (e & 3)) * VW + 32 * i + l32];
-                    o[i] = mfma_split(split3<false>(vs), bp, o[i]);
+                    range.add(vs);
+                    o[i] = mfma_split(split3(vs), bp, o[i]);
                 }
             }
         } else {
@@ -431,7 +443,12 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
     }
     if constexpr (SPLIT) {
 #pragma unroll
-        for (int kk = 0; kk < D / 16; ++kk) qsp[kk] = split3_row(qreg[2 * kk], qreg[2 * kk + 1]);
+        for (int kk = 0; kk < D / 16; ++kk) {
+            const f32x4 u = __builtin_bit_cast(f32x4, qreg[2 * kk]), v = __builtin_bit_cast(f32x4, qreg[2 * kk + 1]);
+            float x[8] = {u[0], u[1], u[2], u[3], v[0], v[1], v[2], v[3]};
+            range.add(x);
+            qsp[kk] = split3(x);
+        }
     }
     sync_tiles();
     if (n_w > 0) {
@@ -499,6 +516,8 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
         constexpr int NF = NO + 3;         // + running max, lane-partial sum, raw max
         static_assert((KS - 1) * 4 * NF * 64 * 4 <= (KS - 1) * C::SMEM_ELEMS * (int)sizeof(T),
                       "split parts fit the other splits' tile buffers");
+        __shared__ __attribute__((aligned(16))) unsigned flags[8];
+        if constexpr (SPLIT) put_odd(flags, range, wg, lane);
         float* mg = reinterpret_cast<float*>(smem + C::SMEM_ELEMS);
         auto at = [&](int s2, int f) FA_INLINE { return mg + (((s2 - 1) * 4 + w) * NF + f) * 64 + lane; };
         if (sp > 0) {
@@ -511,6 +530,12 @@ __global__ __launch_bounds__(256 * KS * QG, KS == 1 && QG == 1 && D <= 128 ? 2 :
             *at(sp, NO + 2) = m_raw;
         }
         lds_barrier();
+        if constexpr (SPLIT) {
+            if (any_odd<8>(flags)) {
+                if (tid == 0) reinterpret_cast<unsigned*>(p.lse)[(int64_t)(b * p.H + h) * p.Sq + q0] = kRedo;
+                return;
+            }
+        }
         if (sp == 0) {
             float mm = m_run;
 #pragma unroll
@@ -976,16 +1001,22 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
             return hipGetLastError();
         }
     }
-    // grids that fill the CUs; smaller ones split the key loop (below), where
-    // the two forms take the same time and the split sums are more accurate
+    // fp32: pieces, by fwd32_kernel on grids that fill the CUs and by the
+    // key-split fwd_kernel on smaller ones (where the two take the same time and
+    // the split sums are more accurate); then the rows that they leave
     if constexpr (Elem<T>::kF32 && std::is_void<TB>::value) {
+        using C = FwdCfg<T, D>;
+        static_assert(F32Cfg<D>::BM == C::BM, "same query blocks");
         P q = p;
-        q.n_qtiles = (p.Sq + F32Cfg<D>::BM - 1) / F32Cfg<D>::BM;
+        q.n_qtiles = (p.Sq + C::BM - 1) / C::BM;
         const int64_t nb = (int64_t)q.n_qtiles * p.H * p.B;
-        if (nb >= 256) {
+        if (nb <= 0) return hipSuccess;
+        if (nb < 256 && p.Sk > C::BN)
+            hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, 2, 1, P>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s, q);
+        else
             hipLaunchKernelGGL((fwd32_kernel<D, CAUSAL, DROPOUT>), dim3((unsigned)nb), dim3(F32Cfg<D>::NT), 0, s, q);
-            return hipGetLastError();
-        }
+        hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, 1, 1, P>), dim3((unsigned)nb), dim3(C::NT), 0, s, q);
+        return hipGetLastError();
     }
     using C = FwdCfg<T, D>;
     // a 16-bit bias without dropout, bias rows of whole 16-byte chunks: staged
