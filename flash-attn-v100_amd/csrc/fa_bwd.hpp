@@ -2460,8 +2460,8 @@ inline bool dkdv8_runs(const BwdParams& p) {
         const int64_t nb = (int64_t)((p.Sk + DkdvCfg<T, D>::BK - 1) / DkdvCfg<T, D>::BK) * p.Hkv * p.B;
         const bool fill1 = BIAS && CAUSAL && p.dbias != nullptr && p.dbias_zero_fill == 1;
         const int seen = p.Sq < p.Sk ? p.Sq : p.Sk;
-        const bool chain = CAUSAL && (nb <= 256 || (nb <= 400 && seen >= (D > 64 ? 1536 : 700)) ||
-                                      (D == 64 && nb <= 512 && seen >= 2048));
+        const bool chain = CAUSAL && (nb <= 256 || (seen >= (D > 64 ? 1536 : 700) &&
+                                                    causal_chain_grid(nb, (int64_t)p.Hkv * p.B, D == 64 && seen >= 2048)));
         return nb > 0 && (nb < 256 || BIAS || chain) && !fill1;
     }
     return false;
@@ -2488,12 +2488,15 @@ inline bool dq_pp_runs(const BwdParams& p) {
 // and with it (bf16; workgroups, keys): D = 64 (384, 4096) 184 / 164, (512, 4096)
 // 171 / 167, (384, 1024) 51.1 / 53.6; D = 128 (384, 2048) 133 / 127, (384, 1024)
 // 80.6 / 86.0; D = 32 (256, 512) 23.8 / 23.5, (256, 4096) 119 / 110, (512, 2048)
-// 70.4 / 70.1, (512, 1024) 41.5 / 42.6.  256: as bwd_small_kernel's.
-template <bool CAUSAL>
+// 70.4 / 70.1, (512, 1024) 41.5 / 42.6, where two of its workgroups fit a CU and
+// uneven grids gain too ((400, 2048) 79 / 76).  256: as bwd_small_kernel's.
+template <int D, bool CAUSAL>
 inline bool dq_splits_keys(const BwdParams& p, int64_t nb, bool plain) {
     if (nb < 256) return true;
     const int seen = p.Sq < p.Sk ? p.Sq : p.Sk;
-    return CAUSAL && plain && (nb == 256 || (nb <= 512 && seen >= 2048));
+    if (!CAUSAL || !plain) return false;
+    if (nb == 256) return true;
+    return seen >= 2048 && (D == 32 ? nb <= 512 : causal_chain_grid(nb, (int64_t)p.H * p.B, D == 64));
 }
 
 // Whether the whole backward runs as the delta pre-pass plus bwd_small_kernel
@@ -2638,7 +2641,7 @@ hipError_t launch_bwd_t(const P& p0, int stage, hipStream_t s) {
         // split the key loop in two inside the workgroup (as the forward does)
         // where two splits' tiles fit the LDS
         if constexpr (!F32_PLAIN && 2 * C::SMEM_BYTES <= 160 * 1024) {
-            if (!done && nb > 0 && dq_splits_keys<CAUSAL>(p, nb, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
+            if (!done && nb > 0 && dq_splits_keys<D, CAUSAL>(p, nb, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
                 hipLaunchKernelGGL((dq_kernel<T, D, CAUSAL, DROPOUT, TB, 2, P>), dim3((unsigned)nb), dim3(C::NT * 2), 0, s,
                                    p, nq);
                 done = true;

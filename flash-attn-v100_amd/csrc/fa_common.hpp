@@ -517,6 +517,24 @@ __device__ FA_INLINE inline int2 tile_order(int n_tiles) {
     return tile_order<SLOTS, FIT>(n_tiles, (int)blockIdx.x, (int)gridDim.x);
 }
 
+// Whether a causal grid of `nb` (above 256) workgroups over `slices` (batch,
+// head) slices gains from a form that runs one workgroup per CU with its chains
+// halved: while an XCD's share is not much above its 32 CUs, or while whole
+// slices divide evenly over the 8 XCDs, up to one and a half (`two`: two)
+// workgroups per CU.  Slices that straddle XCDs leave some of them the long
+// chains of several.  Time ratio, with the form to without, bf16, forward /
+// backward at D = 64 and D = 128 (queries x slices):
+//   (1536 x 22) 0.99 / 0.94, 1.00 / 0.84; (2048 x 17) 0.76 / 0.81, 0.89 / 0.75;
+//   (2048 x 24) 0.85 / 0.86, 0.95 / 0.79; (3000 x 16) 0.81 / 0.84, 0.87 / 0.75;
+//   uneven past 288: (3000 x 13) 1.00 / 1.03, 1.13 / 0.92; (3000 x 15) 1.11 /
+//   1.14, 1.23 / 1.04; (1024 x 44) bwd 1.05; (2048 x 25) 1.10 / 1.19, 1.24 /
+//   1.09; but (2048 x 20) 0.77 / 0.82, 0.89 / 0.76
+//   even, two per CU: (2048 x 32) 0.97 / 0.94, 1.00 / 1.00; (4096 x 16) 0.88 /
+//   0.91, 0.94 / 1.00
+inline bool causal_chain_grid(int64_t nb, int64_t slices, bool two) {
+    return nb <= 288 || (slices % 8 == 0 && nb <= (two ? 512 : 384));
+}
+
 // (batch, head) of slice s of the B x NH slices: batch-major (s = b NH + h),
 // or head-major (s = h B + b) for a kernel that reads a bias shared by the
 // batches (batch stride 0): a group of slices (tile_order) then holds batches

@@ -974,14 +974,15 @@ inline bool fwd_pp_wanted(const FwdParams& p, bool causal) {
 // 12.7 / 12.1, (256, 2048) 29.3 / 24.7, (384, 1024) 19.1 / 20.4, (384, 2048)
 // 30.8 / 26.9, (384, 4096) 76 / 57, (512, 2048) 32.8 / 32.1; D = 128 (256, 1024)
 // 24.9 / 24.6, (384, 2048) 46.1 / 44.3, (512, 2048) 50.7 / 53.3, (512, 4096)
-// 91.6 / 88.0; full rows of one length lose 5-30% ((384, 1024) 28.8 / 32.8).
+// 91.6 / 88.0; D = 32 (512, 2048) 26.4 / 27.8, (512, 4096) 45.2 / 41.3; full rows
+// of one length lose 5-30% ((384, 1024) 28.8 / 32.8).
 template <int D, bool CAUSAL>
-inline bool fwd_splits_keys(int64_t nblocks, int Sq, int Sk, bool plain) {
+inline bool fwd_splits_keys(int64_t nblocks, int64_t slices, int Sq, int Sk, bool plain) {
     if (nblocks < 256) return true;
     if (!CAUSAL || !plain) return false;
     const int keys = Sq < Sk ? Sq : Sk;  // that the last query sees
     if (nblocks == 256) return keys >= (D > 64 ? 1024 : 512);
-    return nblocks <= 512 && keys >= (D > 64 && nblocks > 400 ? 4096 : 2048);
+    return keys >= 2048 && causal_chain_grid(nblocks, slices, keys >= (D == 64 ? 2048 : 4096));
 }
 
 template <typename T, int D, bool CAUSAL, int DROPOUT, typename TB, typename P>
@@ -1061,7 +1062,7 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
     constexpr int KS_SMALL = (!Elem<T>::kF32 && D == 32 && DROPOUT == 0 && std::is_void<TB>::value) ? 4 : 2;
     // (D = 256: one workgroup's tiles take most of the LDS, no split)
     if constexpr (D <= 128) {
-        if (fwd_splits_keys<D, CAUSAL>(nblocks, p.Sq, p.Sk, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
+        if (fwd_splits_keys<D, CAUSAL>(nblocks, (int64_t)p.H * p.B, p.Sq, p.Sk, DROPOUT == 0 && std::is_void<TB>::value) && p.Sk > C::BN) {
             hipLaunchKernelGGL((fwd_kernel<T, D, CAUSAL, DROPOUT, TB, KS_SMALL, 1, P>), dim3((unsigned)nblocks),
                                dim3(C::NT * KS_SMALL), 0, s, q);
             return hipGetLastError();

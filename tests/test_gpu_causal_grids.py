@@ -20,7 +20,9 @@ CASES = [
     (2, 1000, 1000, 16, 16, 128, torch.bfloat16),  # 256 / 256
     (3, 1024, 1024, 16, 4, 128, torch.float16),   # 384 / 96: grouped heads
     (1, 1600, 1600, 24, 24, 128, torch.bfloat16),  # 312 / 312: 8-wave dK/dV
-    (1, 2100, 2100, 20, 20, 64, torch.float16),   # 340 / 340: long chains, key-split dQ and forward
+    (1, 2100, 2100, 20, 20, 64, torch.float16),   # 340 / 340: long chains, slices that straddle XCDs
+    (2, 2050, 2050, 8, 8, 64, torch.float16),     # 272 / 272: the same with key-split dQ and forward
+    (1, 2100, 2100, 24, 24, 64, torch.bfloat16),  # 408 / 408: whole slices per XCD
     (1, 2048, 2304, 32, 32, 64, torch.bfloat16),  # 512 / 576: the last of the rules, keys no query sees
     (1, 2049, 2049, 32, 32, 32, torch.bfloat16),  # 544: past them
     (2, 512, 512, 32, 32, 32, torch.float16),     # 256 at D = 32
