@@ -400,7 +400,10 @@ bool decode_plan(const fa_fwd_args* a, fa::FwdParams& p) {
     if (a->dtype == FA_DTYPE_F32 || a->head_dim > 128 || a->bias || a->dropout_p > 0.f) return false;
     const bool causal = a->causal != 0;
     const int D = a->head_dim;
-    const int64_t rows = (int64_t)(a->num_heads / a->num_heads_kv) * a->seqlen_q;
+    // a causal tile holds rows of one head: it ends at its last query's keys, and
+    // what lies behind them (infinities, NaN) meets no row of another head
+    const int64_t sq = causal ? ((int64_t)a->seqlen_q + 31) / 32 * 32 : a->seqlen_q;
+    const int64_t rows = (int64_t)(a->num_heads / a->num_heads_kv) * sq;
     const int64_t keys = causal ? std::min(a->seqlen_q, a->seqlen_k) : a->seqlen_k;  // that the last query sees
     const int64_t n_rt = (rows + 31) / 32;
     // (rows x batch x KV heads below 2^30 here: no product of this plan overflows)
@@ -441,6 +444,7 @@ bool decode_plan(const fa_fwd_args* a, fa::FwdParams& p) {
         }
     }
     p.dec_rt = (int)n_rt;
+    p.dec_sq = (int)sq;
     p.dec_splits = best;
     return true;
 }

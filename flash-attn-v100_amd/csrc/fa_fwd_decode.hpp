@@ -7,7 +7,8 @@
 // group reads its K / V again, and a key loop, a serial chain of tile
 // latencies, stays inside one workgroup.  Here
 //   * the rows of a workgroup (32) are the (query head of the KV group, query)
-//     pairs of one (batch, KV head): K / V are read once for the whole group;
+//     pairs of one (batch, KV head): K / V are read once for the whole group
+//     (with a causal mask, 32 queries of one head);
 //   * the keys are split over dec_splits workgroups, and inside one over its 4
 //     waves: wave w walks the 64-key tiles t0 + w, t0 + w + 4, ...;
 //   * each wave copies its tiles into its own LDS region (direct-to-LDS), so
@@ -65,19 +66,15 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
     const T* __restrict__ kbase = (const T*)p.k + b * p.k_sb + hk * p.k_sh;
     const T* __restrict__ vbase = (const T*)p.v + b * p.v_sb + hk * p.v_sh;
     // ---- this lane's row: (query head g of the group, query i) ----
-    const int rows = p.group * p.Sq;
-    const int row = 32 * rt + l32;
-    const bool live = row < rows;
-    const int g = live ? row / p.Sq : 0, i = live ? row - g * p.Sq : 0;
+    const int row = 32 * rt + l32, rg = row / p.dec_sq;
+    const bool live = rg < p.group && row - rg * p.dec_sq < p.Sq;
+    const int g = live ? rg : 0, i = live ? row - rg * p.dec_sq : 0;
     const int h = hk * p.group + g;
-    // key tiles that some row of the unit sees (rows that cross into the next
-    // head end at a head's last query)
+    // key tiles that some row of the unit sees (causal: the unit's rows are
+    // consecutive queries of one head)
     int nt = (p.Sk + BN - 1) / BN;
-    if (CAUSAL) {
-        const int r0 = 32 * rt, r1 = min(r0 + 31, rows - 1);
-        const int i_last = r0 / p.Sq == r1 / p.Sq ? r1 % p.Sq : p.Sq - 1;
-        nt = min(nt, i_last / BN + 1);
-    }
+    const int i_first = CAUSAL ? (32 * rt) % p.dec_sq : 0;
+    if (CAUSAL) nt = min(nt, min(i_first + 31, p.Sq - 1) / BN + 1);
     const int t0 = (int)((int64_t)nt * split / p.dec_splits), t1 = (int)((int64_t)nt * (split + 1) / p.dec_splits);
 
     T* Ks = smem + w * C::REGION;
@@ -118,11 +115,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 2 : 1) void fwd_decode_kernel(const 
     const float c = p.scale_log2;
 
     // causal: tiles before n_um are whole for every row of the unit
-    int n_um = 0;
-    if (CAUSAL) {
-        const int r0 = 32 * rt, r1 = min(r0 + 31, rows - 1);
-        n_um = r0 / p.Sq == r1 / p.Sq ? (r0 % p.Sq + 1) / BN : 0;
-    }
+    const int n_um = CAUSAL ? (i_first + 1) / BN : 0;
     int t = t0 + w;
     copy_k(t);
     copy_v(t);
@@ -284,8 +277,8 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const P p, const int n
     const int r = gid / TPR, col = (gid % TPR) * 4;
     if (r >= n_rows) return;
     // row r = ((b Hkv + hk) group + g) Sq + i, i.e. (b, h, i) in order
-    const int rows = p.group * p.Sq;
-    const int bk = r / rows, rr = r - bk * rows;
+    const int bk = r / (p.group * p.Sq), gi = r - bk * (p.group * p.Sq);
+    const int rr = gi / p.Sq * p.dec_sq + gi % p.Sq;
     const int64_t base = ((int64_t)(bk * p.dec_rt + (rr >> 5)) * p.dec_splits) * 32 + (rr & 31);
     float mm = -1e30f, m_raw = -INFINITY;
     for (int x = 0; x < p.dec_splits; ++x) {

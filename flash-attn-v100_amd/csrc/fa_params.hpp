@@ -49,10 +49,11 @@ struct FwdParams {
     int bias_span;  // bytes of one (batch, head) slice: ((Sq - 1) * ss + Sk) * elem
     // few-row forward (fa_fwd_decode.hpp), taken when dec_splits > 0: its units
     // are the 32-row tiles of the (query head of the group, query) rows of each
-    // (batch, KV head), dec_rt per (batch, KV head); with dec_splits > 1 the
+    // (batch, KV head), dec_rt per (batch, KV head), a head's rows dec_sq apart
+    // (Sq, or with a causal mask Sq rounded up to whole tiles); with dec_splits > 1 the
     // parts of a unit's key splits go to the caller's workspace (per row 4
     // floats of statistics, and D floats of O)
-    int dec_splits, dec_rt;
+    int dec_splits, dec_rt, dec_sq;
     float* dec_stat;
     float* dec_part;
     // columns of q, k, v and o that exist (a multiple of 8; 0: all D): a head

@@ -71,3 +71,17 @@ def test_split_plan_needs_its_workspace():
     assert lib.fa_fwd_workspace_size(ctypes.byref(short)) == 0
     assert lib.fa_fwd_ws(ctypes.byref(short), None, 0, _lib._stream(q)) == 0
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_causal_rows_do_not_meet_later_keys(D):
+    # grouped heads whose length is no multiple of the 32-row tiles: NaN in the
+    # keys and values of the last rows reaches no row before their 64-key tile
+    print(f"case: few rows, later keys {D}", flush=True)
+    g = torch.Generator("cuda").manual_seed(D)
+    q, k, v = (torch.randn(2, 200, h, D, generator=g, device="cuda").to(torch.bfloat16) for h in (8, 2, 2))
+    want = _lib.fwd(q, k, v, True, D ** -0.5)
+    k[:, 150:], v[:, 150:] = float("nan"), float("nan")
+    got = _lib.fwd(q, k, v, True, D ** -0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0][:, :128], want[0][:, :128]) and torch.equal(got[1][:, :, :128], want[1][:, :, :128])
