@@ -209,22 +209,42 @@ PyObject* host_bwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(fa_fwd_workspace_size, fa_fwd_ws, fa_fwd_cols, fa_bwd_workspace_size,
-//      fa_bwd, fa_bwd_cols): their addresses in the loaded kernel library
+// bind(fa_abi_version, sizeof(fa_fwd_args), sizeof(fa_bwd_args),
+//      fa_fwd_workspace_size, fa_fwd_ws, fa_fwd_cols, fa_bwd_workspace_size,
+//      fa_bwd, fa_bwd_cols): addresses in the loaded kernel library, and the
+// struct sizes of the layer that binds it.  Refused where the library or that
+// layer speaks another version than this module was compiled for: the structs
+// carry device pointers.
 PyObject* host_bind(PyObject*, PyObject* const* x, Py_ssize_t n) {
-    if (n != 6) {
-        PyErr_SetString(PyExc_TypeError, "bind takes six addresses");
+    if (n != 9) {
+        PyErr_SetString(PyExc_TypeError, "bind takes seven addresses and two sizes");
         return nullptr;
     }
-    void* p[6];
-    for (int i = 0; i < 6; ++i) p[i] = PyLong_AsVoidPtr(x[i]);
+    void* p[7];
+    for (int i = 0; i < 7; ++i) {
+        p[i] = PyLong_AsVoidPtr(x[i == 0 ? 0 : i + 2]);
+        if (PyErr_Occurred()) return nullptr;
+        if (!p[i]) {
+            PyErr_SetString(PyExc_ValueError, "bind: null address");
+            return nullptr;
+        }
+    }
+    const size_t sizes[2] = {PyLong_AsSize_t(x[1]), PyLong_AsSize_t(x[2])};
     if (PyErr_Occurred()) return nullptr;
-    p_fwd_ws_size = (decltype(p_fwd_ws_size))p[0];
-    p_fwd_ws = (decltype(p_fwd_ws))p[1];
-    p_fwd_cols = (decltype(p_fwd_cols))p[2];
-    p_bwd_ws_size = (decltype(p_bwd_ws_size))p[3];
-    p_bwd = (decltype(p_bwd))p[4];
-    p_bwd_cols = (decltype(p_bwd_cols))p[5];
+    const int32_t version = ((decltype(&fa_abi_version))p[0])();
+    if (version != FA_ABI_VERSION || sizes[0] != sizeof(fa_fwd_args) || sizes[1] != sizeof(fa_bwd_args)) {
+        PyErr_Format(PyExc_RuntimeError,
+                     "fa_host was built for ABI version %d with argument structs of %zu and %zu bytes; the library has "
+                     "version %d, the binding %zu and %zu bytes",
+                     FA_ABI_VERSION, sizeof(fa_fwd_args), sizeof(fa_bwd_args), (int)version, sizes[0], sizes[1]);
+        return nullptr;
+    }
+    p_fwd_ws_size = (decltype(p_fwd_ws_size))p[1];
+    p_fwd_ws = (decltype(p_fwd_ws))p[2];
+    p_fwd_cols = (decltype(p_fwd_cols))p[3];
+    p_bwd_ws_size = (decltype(p_bwd_ws_size))p[4];
+    p_bwd = (decltype(p_bwd))p[5];
+    p_bwd_cols = (decltype(p_bwd_cols))p[6];
     Py_RETURN_NONE;
 }
 

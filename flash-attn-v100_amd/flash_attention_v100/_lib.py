@@ -91,6 +91,21 @@ ERR_SCRATCH = -14
 _lib = None
 
 
+def _check_library(lib, path: str) -> None:
+    """The version this module mirrors, with every function of it (functions are
+    added without a new version)."""
+    if hasattr(lib, "fa_abi_version"):
+        lib.fa_abi_version.restype = ctypes.c_int32
+        lib.fa_abi_version.argtypes = []
+        v = lib.fa_abi_version()
+        if v != ABI_VERSION:
+            raise FlashAttentionExtensionError(f"{path} has ABI version {v}, expected {ABI_VERSION}")
+    missing = [n for n in EXPORTS if not hasattr(lib, n)]
+    if missing:
+        raise FlashAttentionExtensionError(f"{path} has no {', '.join(missing)}; build it with "
+                                           "`python flash-attn-v100_amd/build.py`")
+
+
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Load (once) and type the library; raises FlashAttentionExtensionError."""
     global _lib
@@ -104,9 +119,8 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         lib = ctypes.CDLL(path)
     except OSError as e:  # pragma: no cover - depends on the machine
         raise FlashAttentionExtensionError(f"cannot load {path}: {e}") from e
+    _check_library(lib, path)
     P = ctypes.POINTER
-    lib.fa_abi_version.restype = ctypes.c_int32
-    lib.fa_abi_version.argtypes = []
     lib.fa_strerror.restype = ctypes.c_char_p
     lib.fa_strerror.argtypes = [ctypes.c_int32]
     lib.fa_fwd_check.restype = ctypes.c_int32
@@ -137,14 +151,24 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
                                     ctypes.c_void_p]
     lib.fa_rand.restype = ctypes.c_int32
     lib.fa_rand.argtypes = [ctypes.c_uint64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]
-    v = lib.fa_abi_version()
-    if v != ABI_VERSION:
-        raise FlashAttentionExtensionError(f"{path} has ABI version {v}, expected {ABI_VERSION}")
     _lib = lib
     return lib
 
 
 _host_mod = None
+
+
+def _bind_host(mod, lib) -> None:
+    """Give the host module the library's functions; refused by the module where
+    it was compiled for another ABI version or other struct layouts."""
+    addr = [ctypes.cast(f, ctypes.c_void_p).value for f in (
+        lib.fa_abi_version, lib.fa_fwd_workspace_size, lib.fa_fwd_ws, lib.fa_fwd_cols, lib.fa_bwd_workspace_size,
+        lib.fa_bwd, lib.fa_bwd_cols)]
+    try:
+        mod.bind(addr[0], ctypes.sizeof(FwdArgs), ctypes.sizeof(BwdArgs), *addr[1:])
+    except RuntimeError as e:
+        raise FlashAttentionExtensionError(f"{HOST_PATH}: {e}; build both with "
+                                           "`python flash-attn-v100_amd/build.py`") from e
 
 
 def _host():
@@ -162,9 +186,7 @@ def _host():
         loader.exec_module(mod)
     except ImportError as e:  # pragma: no cover - depends on the machine
         raise FlashAttentionExtensionError(f"cannot load {HOST_PATH}: {e}") from e
-    mod.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
-        lib.fa_fwd_workspace_size, lib.fa_fwd_ws, lib.fa_fwd_cols, lib.fa_bwd_workspace_size, lib.fa_bwd,
-        lib.fa_bwd_cols)))
+    _bind_host(mod, lib)
     _host_mod = mod
     return mod
 
