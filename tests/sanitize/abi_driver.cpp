@@ -295,6 +295,114 @@ static void bwd_paths() {
     t = a; t.dropout_p = 3.f; CHECK(fa_bwd_static(&t, nullptr) == FA_ERR_DROPOUT);
 }
 
+// The few-row forward's plan: which calls take it, that its parts fit exactly
+// the workspace it asks for, and what a missing workspace gives.
+static void few_rows() {
+    int taken = 0, split = 0;
+    for (int D : {32, 64, 128})
+        for (int causal = 0; causal < 2; ++causal)
+            for (int group : {1, 3, 8})
+                for (int Sq : {1, 5, 31, 32, 33, 200, 1500})
+                    for (int Sk : {1, 64, 65, 300, 4096, 30000})
+                        for (int B : {1, 3, 70}) {
+                            // (no buffer is read: one of any size stands for all)
+                            fa_fwd_args a = make_fwd(1, 1, 1, 2 * group, 2, D, FA_DTYPE_BF16, causal);
+                            a.batch = B;
+                            a.seqlen_q = Sq;
+                            a.seqlen_k = Sk;
+                            const size_t n = fa_fwd_workspace_size(&a);
+                            CHECK(fa_fwd(&a, nullptr) == FA_OK);
+                            CHECK(g_stub.fwd.dec_splits == 0);  // without a workspace: the other kernels
+                            char* ws = n ? (char*)alloc(n) : nullptr;
+                            CHECK(fa_fwd_ws(&a, ws, n, nullptr) == FA_OK);
+                            const fa::FwdParams p = g_stub.fwd;
+                            CHECK((n > 0) == (p.dec_splits > 1));
+                            if (p.dec_splits == 0) continue;
+                            ++taken;
+                            // the tiles hold every row; causal: whole tiles of one head
+                            CHECK(p.dec_sq >= Sq && p.dec_sq < Sq + 32 && (!causal || p.dec_sq % 32 == 0));
+                            CHECK((int64_t)p.dec_rt * 32 >= (int64_t)group * p.dec_sq &&
+                                  (int64_t)(p.dec_rt - 1) * 32 < (int64_t)group * p.dec_sq);
+                            const int keys = causal && Sq < Sk ? Sq : Sk;
+                            CHECK(p.dec_splits <= (keys + 63) / 64);
+                            if (p.dec_splits == 1) continue;
+                            ++split;
+                            const size_t rows = (size_t)B * 2 * p.dec_rt * p.dec_splits * 32;
+                            CHECK(p.dec_stat == (float*)ws && p.dec_part == p.dec_stat + rows * 4);
+                            CHECK((char*)(p.dec_part + rows * D) == ws + n);
+                            const int calls = g_stub.fwd_calls;
+                            CHECK(fa_fwd_ws(&a, nullptr, n, nullptr) == FA_ERR_WORKSPACE);
+                            CHECK(fa_fwd_ws(&a, ws, n - 1, nullptr) == FA_ERR_WORKSPACE);
+                            CHECK(fa_fwd_ws(&a, ws + 4, n, nullptr) == FA_ERR_WORKSPACE);
+                            CHECK(g_stub.fwd_calls == calls);
+                        }
+    CHECK(taken > 100 && split > 50);
+    // not for float32, dropout, a bias or head dim 256; nothing for invalid calls
+    fa_fwd_args a = make_fwd(1, 1, 1, 8, 2, 128, FA_DTYPE_F16, 0), t = a;
+    a.seqlen_k = t.seqlen_k = 16384;
+    CHECK(fa_fwd_workspace_size(&a) > 0 && fa_fwd_workspace_size(nullptr) == 0);
+    t.dropout_p = 0.1f; CHECK(fa_fwd_workspace_size(&t) == 0);
+    t = a; t.dtype = FA_DTYPE_F32; CHECK(fa_fwd_workspace_size(&t) == 0);
+    t = a; t.head_dim = 256; CHECK(fa_fwd_workspace_size(&t) == 0);
+    t = a; t.bias = alloc(64); CHECK(fa_fwd_workspace_size(&t) == 0);
+    t = a; t.num_heads = 7; CHECK(fa_fwd_workspace_size(&t) == 0 && fa_fwd_ws(&t, nullptr, 0, nullptr) == FA_ERR_HEADS);
+    t = a; t.batch = 0; CHECK(fa_fwd_workspace_size(&t) == 0 && fa_fwd_ws(&t, nullptr, 0, nullptr) == FA_OK);
+    // sizes at the limits: no overflow in the plan (rows, units, workspace)
+    for (int B : {1, 1 << 16, 1 << 20})
+        for (int Sq : {1, 1 << 14, (1 << 14) + 1, (1 << 28) - 1})
+            for (int Sk : {0, 1, (1 << 28) - 1})
+                for (int hkv : {1, 1 << 10, 1 << 16})
+                    for (int group : {1, 1 << 14}) {
+                        t = a;
+                        t.batch = B;
+                        t.seqlen_q = Sq;
+                        t.seqlen_k = Sk;
+                        t.num_heads_kv = hkv;
+                        t.num_heads = hkv * group;
+                        for (int causal = 0; causal < 2; ++causal) {
+                            t.causal = causal;
+                            const size_t n = fa_fwd_workspace_size(&t);
+                            CHECK(n < (size_t)1 << 40);
+                            const int32_t st = fa_fwd_ws(&t, n ? (void*)a.q : nullptr, n, nullptr);
+                            CHECK(st == FA_OK || st == FA_ERR_TOO_LARGE);
+                            if (st != FA_OK || g_stub.fwd.dec_splits == 0 || Sq == 0) continue;
+                            // workgroups, and threads of the combining kernel, in 32 bits
+                            CHECK((int64_t)B * hkv * g_stub.fwd.dec_rt * g_stub.fwd.dec_splits < (int64_t)1 << 31);
+                            if (g_stub.fwd.dec_splits > 1)
+                                CHECK((int64_t)B * t.num_heads * Sq * (a.head_dim / 4) < (int64_t)1 << 31);
+                        }
+                    }
+}
+
+// Head dims between the compiled ones: the columns that reach the kernels, and
+// what is refused.
+static void columns() {
+    for (int D : {64, 128, 256})
+        for (int cols = -8; cols <= 264; ++cols) {
+            fa_fwd_args a = make_fwd(1, 40, 40, 2, 1, D, FA_DTYPE_F16, 1);
+            fa_bwd_args b = make_bwd(1, 40, 40, 2, 1, D, FA_DTYPE_BF16, 0);
+            const size_t n = fa_bwd_workspace_size(&b);
+            void* ws = alloc(n);
+            const bool ok = cols > D / 2 && cols <= D && cols % 8 == 0;
+            const int fc = g_stub.fwd_calls, bc = g_stub.bwd_calls;
+            CHECK(fa_fwd_cols(&a, cols, nullptr, 0, nullptr) == (ok ? FA_OK : FA_ERR_HEAD_DIM));
+            CHECK(fa_bwd_cols(&b, cols, ws, n, nullptr) == (ok ? FA_OK : FA_ERR_HEAD_DIM));
+            CHECK(g_stub.fwd_calls == fc + ok && g_stub.bwd_calls == bc + ok);
+            if (!ok) continue;
+            const int want = cols == D ? 0 : cols;
+            CHECK(g_stub.fwd.head_cols == want && g_stub.bwd.head_cols == want && g_stub.D == D);
+            CHECK(fa_bwd_cols(&b, cols, nullptr, n, nullptr) == FA_ERR_WORKSPACE);
+            CHECK(fa_bwd_cols(&b, cols, ws, n - 4, nullptr) == FA_ERR_WORKSPACE);
+        }
+    CHECK(fa_fwd_cols(nullptr, 72, nullptr, 0, nullptr) == FA_ERR_NULL_ARG);
+    fa_fwd_args a = make_fwd(1, 40, 40, 2, 2, 128, FA_DTYPE_F16, 1), t = a;
+    t.dropout_p = 0.1f; CHECK(fa_fwd_cols(&t, 72, nullptr, 0, nullptr) == FA_ERR_HEAD_DIM);
+    t = a; t.dtype = FA_DTYPE_F32; CHECK(fa_fwd_cols(&t, 72, nullptr, 0, nullptr) != FA_OK);
+    t = make_fwd(1, 40, 40, 2, 2, 32, FA_DTYPE_F16, 1); CHECK(fa_fwd_cols(&t, 24, nullptr, 0, nullptr) == FA_ERR_HEAD_DIM);
+    t = a; t.bias = alloc(40 * 40 * 2); t.bias_dtype = FA_DTYPE_F16; t.bias_stride[2] = 40;
+    CHECK(fa_fwd_cols(&t, 72, nullptr, 0, nullptr) == FA_ERR_HEAD_DIM);
+}
+
 // The range of a tile descriptor never reaches the row behind the last valid
 // one, whatever columns exist and however close the rows follow, and never
 // loses a valid element: every head dim that runs at a wider compiled one.
@@ -327,6 +435,8 @@ int main() {
     fwd_valid();
     fwd_rejects();
     bwd_paths();
+    few_rows();
+    columns();
     tile_ranges();
     misc();
     for (void* p : g_bufs) std::free(p);
