@@ -20,7 +20,8 @@
 // 7.5e-7, 7.3e-7), causal 2.6e-7, 3.6e-7, 3.6e-7, 3.0e-7 (3.3e-7, 4.8e-7, 4.9e-7,
 // 4.2e-7).
 // Measured (forward / dQ and dK/dV, us; before: on v_mfma_f32_32x32x2_f32; the
-// kernels for marked rows, of which there are none here, are 1 to 2 of each):
+// three launches for marked rows, of which there are none here, take 4 to 5 each
+// on 1000 workgroups, 1.5 on few):
 // 8 x 1000 x 16 heads of 64, full: 288 / 916 -> 203 / 635; causal with dropout,
 // heads of 32, 64, 128: 225 / 324, 307 / 595, 457 / 1213 -> 156 / 229, 199 /
 // 405, 361 / 993; 4 x 1024 x 16 heads of 128, full: 262 / 982 -> 199 / 686.
