@@ -528,7 +528,8 @@ __device__ FA_INLINE inline int2 tile_order(int n_tiles) {
 //   (2048 x 24) 0.85 / 0.86, 0.95 / 0.79; (3000 x 16) 0.81 / 0.84, 0.87 / 0.75;
 //   uneven past 288: (3000 x 13) 1.00 / 1.03, 1.13 / 0.92; (3000 x 15) 1.11 /
 //   1.14, 1.23 / 1.04; (1024 x 44) bwd 1.05; (2048 x 25) 1.10 / 1.19, 1.24 /
-//   1.09; but (2048 x 20) 0.77 / 0.82, 0.89 / 0.76
+//   1.09; but (2048 x 20) 0.77 / 0.82, 0.89 / 0.76 (D = 96: (2048 x
+//   25) 1.18 / 1.26, (2048 x 24) 0.90 / 0.93)
 //   even, two per CU: (2048 x 32) 0.97 / 0.94, 1.00 / 1.00; (4096 x 16) 0.88 /
 //   0.91, 0.94 / 1.00
 inline bool causal_chain_grid(int64_t nb, int64_t slices, bool two) {

@@ -1031,7 +1031,9 @@ hipError_t launch_fwd_t(const P& p, hipStream_t s) {
             // 128-query workgroups, keys): (256, 2048) 55.7 / 34.8, full 57.5 / 34.6,
             // (192, 2048) 48.1 / 33.9, (256, 512) 17.5 / 13.8, (64, 256) 11.1 / 10.1;
             // causal (512, 2048) 58.1 / 46.3, (512, 1024) 32.6 / 29.8, (512, 512)
-            // 20.6 / 21.5; full (512, 1024) 33.0 / 39.1
+            // 20.6 / 21.5, (400, 2048) 68.3 / 57.5, (400, 1024) 39.8 / 36.4; full
+            // (512, 1024) 33.0 / 39.1; D = 32 (256, 2048) 60.3 / 32.0, (64, 256) 10.1 /
+            // 8.3, causal (512, 1024) 30.8 / 26.4, (400, 2048) 71.8 / 50.4
             if constexpr (D <= 64) {
                 P q = p;
                 q.n_qtiles = (p.Sq + C::BM - 1) / C::BM;
